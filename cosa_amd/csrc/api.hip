@@ -272,7 +272,7 @@ int cosahip_create(const cosahip_config* cfg, int device, cosahip_solve** out) {
   const char* vk = getenv("COSAHIP_VISCOUS");
   s->fuse_viscous = vk && strcmp(vk, "fused") == 0;
   s->viscous_faces = !(vk && (strcmp(vk, "march") == 0 || strcmp(vk, "fused") == 0));
-  s->viscous_tile = vk && strcmp(vk, "tile") == 0;
+  s->viscous_tile = !(vk && (strcmp(vk, "march") == 0 || strcmp(vk, "fused") == 0 || strcmp(vk, "faces") == 0));
   const char* jk = getenv("COSAHIP_CIRS_JK");
   s->cirs_jk_chunk = !jk ? 4 : strcmp(jk, "plain") == 0 ? 0 : strcmp(jk, "chunk8") == 0 ? 8 : 4;
   if (device >= 0) {
@@ -449,6 +449,7 @@ static int build_tables(Solve* s, Level& L, const Level* Lc) {
   const int ns = s->par.nsnap;
   for (int k = 0; k < TK_NKIND; k++) L.htile[k].clear();
   plan_cirs_il(s, L);
+  L.kseg = residual_kseg(L.hblk, ns);
   for (int b = 0; b < L.nblocks; b++) {
     const Blk& B = L.hblk[b];
     const ll im = B.imax - 1, jm = B.jmax - 1, km = B.kmax - 1;
@@ -472,9 +473,9 @@ static int build_tables(Solve* s, Level& L, const Level* Lc) {
     add_tiles(L.htile[TK_SHELL], b, ns * (2 * (ll)(B.jmax + 1) * (B.kmax + 1) + im * (2 * (ll)(B.kmax + 1) + 2 * jm)),
               TS);
     add_tiles(L.htile[TK_HALO], b, ns * ((ll)(B.imax + 3) * jm * km + 4 * im * km + 4 * im * jm), TS);
-    add_tiles(L.htile[TK_FUSED], b, residual_tile_items(RT_TI, 7, B.imax, B.jmax, B.kmax, ns), 1);
-    add_tiles(L.htile[TK_FUSED15], b, residual_tile_items(RT_TI, 15, B.imax, B.jmax, B.kmax, ns), 1);
-    add_tiles(L.htile[TK_T32], b, residual_tile_items(32, 7, B.imax, B.jmax, B.kmax, ns), 1);
+    add_tiles(L.htile[TK_FUSED], b, residual_tile_items(RT_TI, 7, L.kseg, B.imax, B.jmax, B.kmax, ns), 1);
+    add_tiles(L.htile[TK_FUSED15], b, residual_tile_items(RT_TI, 15, L.kseg, B.imax, B.jmax, B.kmax, ns), 1);
+    add_tiles(L.htile[TK_T32], b, residual_tile_items(32, 7, L.kseg, B.imax, B.jmax, B.kmax, ns), 1);
     if (Lc) {
       const Blk& C = Lc->hblk[b];
       add_tiles(L.htile[TK_COARSE], b, ns * (ll)(C.imax - 1) * (C.jmax - 1) * (C.kmax - 1), TS);

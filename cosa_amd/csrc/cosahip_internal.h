@@ -91,7 +91,7 @@ enum TileKind {
   TK_COARSE,      // cells of the next coarser level, per block (restriction)
   TK_PROL,        // 2x2x2 prolongation groups 0..imax-1 step 2, per block
   TK_HALO,        // prtest region: interior + face halo strips
-  TK_FUSED,       // fused residual: (31 x 7)-cell (i,j) tiles x 32-plane k segments
+  TK_FUSED,       // fused residual: (31 x 7)-cell (i,j) tiles x kseg-plane k segments
   TK_LINES_I_T,   // (jmax-1)(kmax-1) lines along i, TS per tile (thread per line)
   TK_LINES_IL,    // (jmax-1)(kmax-1) lines along i, il_lpw per tile (whole lines resident in LDS)
   TK_LINES_IV,    // (jmax-1)(kmax-1) lines along i, 256/npde per tile (thread per line and variable)
@@ -100,9 +100,9 @@ enum TileKind {
   TK_FACES_I,     // i faces imax x (jmax-1) x (kmax-1)
   TK_FACES_J,     // j faces (imax-1) x jmax x (kmax-1)
   TK_FACES_K,     // k faces (imax-1) x (jmax-1) x kmax
-  TK_FUSED15,     // residual tiles of 31 x 15 cells x 32-plane k segments (k_residual_tile, TJ = 15)
+  TK_FUSED15,     // residual tiles of 31 x 15 cells x kseg-plane k segments (k_residual_tile, TJ = 15)
   TK_SHELL,       // the halo shell of 0..imax x 0..jmax x 0..kmax (the box without the interior cells)
-  TK_T32,         // residual tiles of 32 x 7 cells x 32-plane k segments (RESID_TILE32_W4, RESID_SVA32)
+  TK_T32,         // residual tiles of 32 x 7 cells x kseg-plane k segments (RESID_TILE32_W4, RESID_SVA32)
   TK_NKIND
 };
 
@@ -193,7 +193,8 @@ struct Level {
   double* work1 = nullptr;    // copy of res for the HB norm
   double* dqc = nullptr;      // SST: (P3, 9, nsnap) cell-centre velocity differences of the stage
   int cirs_mode = 0;          // CIRS i-sweep picked by cosahip_autotune: 0 none, 1 lds, 2 iv, 3 line
-  int resid_mode = RESID_GENERIC;   // inviscid residual kernel (ResidVariant)
+  int resid_mode = RESID_SVA32;   // inviscid residual kernel (ResidVariant)
+  int kseg = 1;               // k-planes per work-group of the residual tiles (residual_kseg)
   int il_lpw = 0;             // k_cirs_il: lines per work-group (0: lines too long for its LDS budget)
   int il_stride = 0;          // k_cirs_il: odd LDS row stride >= the longest i-line of the level
   double* il_rtab = nullptr;  // k_cirs_il: multipliers and reciprocal divisors, 2 il_stride per block
@@ -288,15 +289,17 @@ struct Solve {
   // direction (COSAHIP_RESIDUAL=split in the environment at create time)
   bool split_residual = false;
   int resid_force = -1;   // COSAHIP_RESIDUAL=fused|tile7|tile7reg|tile15|tile7w4|sva7|sva15|sva7w4: that kernel on every level
-  // viscous face fluxes after the inviscid pass of each direction: face
-  // fluxes stored then differenced (default), flux and difference in one
-  // marching kernel (COSAHIP_VISCOUS=march), or fused into the inviscid line
-  // march (COSAHIP_VISCOUS=fused); or the face fluxes of all three
-  // directions stored, then one tile pass for the inviscid fluxes and every
-  // difference (COSAHIP_VISCOUS=tile), all at create time
+  // viscous face fluxes: those of all three directions stored, then one tile
+  // pass for the inviscid fluxes and every difference (default); per
+  // direction after its inviscid line march, stored then differenced
+  // (COSAHIP_VISCOUS=faces) or flux and difference in one marching kernel
+  // (=march); or fused into the inviscid march (=fused), all at create time.
+  // The tile pass has a work-group per 32 x 7 x kseg cells, the marches a
+  // thread per 16-cell segment: on the SST 257 x 65 x 9 O-grid 143 us against
+  // 225 us of a level-1 residual, on the wing (autotuned before) it wins too
   bool fuse_viscous = false;
   bool viscous_faces = true;
-  bool viscous_tile = false;
+  bool viscous_tile = true;
   // CIRS i-sweep: one thread per (line, variable) on levels with fewer than
   // CIRS_IV_MAX_LINES lines along i, one thread per line with LDS-staged
   // chunks on larger ones; COSAHIP_CIRS_I=lds|iv at create time forces one

@@ -252,7 +252,7 @@ __global__ void __launch_bounds__(64) k_h0_last(Par p, int nl, int nblocks, cons
 // ------------------------------------------------------------------------
 // Fused residual, all three directions in one pass (2.5-D blocking).
 // A workgroup of 32 x 8 threads owns FTI x FTJ = 31 x 7 cells of an (i,j)
-// tile and marches k through a segment of up to KSEG planes.  Per plane:
+// tile and marches k through a segment of kseg planes.  Per plane:
 //   - the plane (primitive q, i0-2..i0+FTI+1 x j0-2..j0+FTJ+1, no corners)
 //     is staged in LDS: cell threads deposit their own value from their
 //     k-window, the halo ring is loaded from global memory;
@@ -263,14 +263,15 @@ __global__ void __launch_bounds__(64) k_h0_last(Par p, int nl, int nblocks, cons
 //     the reference's accumulation order (zero, then resid for idir = 1,2,3).
 // Every face flux is computed from the same operands as in the split
 // kernels, so the results are identical.
-constexpr int FTI = 31, FTJ = 7, KSEG = 32;
+constexpr int FTI = 31, FTJ = 7;
 constexpr int PW = FTI + 4, PH = FTJ + 4;
 
 template <typename T>
 __global__ void __launch_bounds__(256) k_residual_fused(Par p, int nl, const Blk* __restrict__ blks,
-                                                        const Tile* __restrict__ tiles, const T* __restrict__ q,
-                                                        const T* __restrict__ si, const T* __restrict__ sj,
-                                                        const T* __restrict__ sk, double* __restrict__ res,
+                                                        const Tile* __restrict__ tiles, int kseg,
+                                                        const T* __restrict__ q, const T* __restrict__ si,
+                                                        const T* __restrict__ sj, const T* __restrict__ sk,
+                                                        double* __restrict__ res,
                                                         const unsigned char* __restrict__ sbc,
                                                         const ll* __restrict__ sbcoff) {
   __shared__ T pl[5][PH][PW];
@@ -280,7 +281,7 @@ __global__ void __launch_bounds__(256) k_residual_fused(Par p, int nl, const Blk
   const Blk b = blks[t.block];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int im = b.imax - 1, jm = b.jmax - 1, km = b.kmax - 1;
-  const int ntx = (im + FTI - 1) / FTI, nty = (jm + FTJ - 1) / FTJ, nks = (km + KSEG - 1) / KSEG;
+  const int ntx = (im + FTI - 1) / FTI, nty = (jm + FTJ - 1) / FTJ, nks = (km + kseg - 1) / kseg;
   int item = t.base;
   const int n = item / (ntx * nty * nks);
   item -= n * (ntx * nty * nks);
@@ -288,7 +289,7 @@ __global__ void __launch_bounds__(256) k_residual_fused(Par p, int nl, const Blk
   item -= ks_i * (ntx * nty);
   const int ty_i = item / ntx, tx_i = item - (item / ntx) * ntx;
   const int i0 = 1 + tx_i * FTI, j0 = 1 + ty_i * FTJ;
-  const int ks = 1 + ks_i * KSEG, ke = min(km, ks + KSEG - 1);
+  const int ks = 1 + ks_i * kseg, ke = min(km, ks + kseg - 1);
   const ll n3 = n3of(b);
   const T* qb = q + b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n;
   double* rb = res + b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n;
@@ -1399,7 +1400,7 @@ hipError_t launch_residual(Solve& s, Level& L, const double* q, double* res) {
     if (rv != RESID_GENERIC) return launch_residual_tile(s, L, rv, L.q32, L.m32[0], L.m32[1], L.m32[2], res);
     if (L.ntile[TK_FUSED])
       hipLaunchKernelGGL(k_residual_fused<float>, grid1(L.ntile[TK_FUSED]), dim3(256), 0, s.stream, s.par, L.nl, L.dblk,
-                         L.tile[TK_FUSED], L.q32, L.m32[0], L.m32[1], L.m32[2], res, L.sbc, L.sbc_doff);
+                         L.tile[TK_FUSED], L.kseg, L.q32, L.m32[0], L.m32[1], L.m32[2], res, L.sbc, L.sbc_doff);
     return hipGetLastError();
   }
   if (!s.split_residual) {
@@ -1411,7 +1412,7 @@ hipError_t launch_residual(Solve& s, Level& L, const double* q, double* res) {
       return launch_residual_tile(s, L, rv, q, L.f[COSAHIP_SI], L.f[COSAHIP_SJ], L.f[COSAHIP_SK], res);
     if (L.ntile[TK_FUSED])
       hipLaunchKernelGGL(k_residual_fused<double>, grid1(L.ntile[TK_FUSED]), dim3(256), 0, s.stream, s.par, L.nl, L.dblk,
-                         L.tile[TK_FUSED], q, L.f[COSAHIP_SI], L.f[COSAHIP_SJ], L.f[COSAHIP_SK], res, L.sbc,
+                         L.tile[TK_FUSED], L.kseg, q, L.f[COSAHIP_SI], L.f[COSAHIP_SJ], L.f[COSAHIP_SK], res, L.sbc,
                          L.sbc_doff);
     return hipGetLastError();
   }

@@ -26,6 +26,8 @@
 //       column i0+tx from LDS, and cell threads compute k-face k+1;
 //   (c) res(c) = ((((0 + Fi(c+1)) - Fi(c)) + Fj(c+1)) - Fj(c)) + Fk(c+1)) - Fk(c),
 //       the reference's accumulation order (zero, then resid for idir = 1, 2, 3).
+#include <algorithm>
+
 #include "flux_face.h"
 #include "kernels.h"
 
@@ -43,7 +45,7 @@ namespace exact {
 
 template <typename T, int TI, int TJ, int ILIM, int FO, int EF, int KW, int MINW>
 __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_tile(Par p, int nl, const Blk* __restrict__ blks,
-                                                                 const Tile* __restrict__ tiles,
+                                                                 const Tile* __restrict__ tiles, int kseg,
                                                                  const T* __restrict__ q, const T* __restrict__ si,
                                                                  const T* __restrict__ sj, const T* __restrict__ sk,
                                                                  double* __restrict__ res,
@@ -58,7 +60,7 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_tile(Par p, in
   const Blk b = blks[t.block];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int im = b.imax - 1, jm = b.jmax - 1, km = b.kmax - 1;
-  const int ntx = (im + TI - 1) / TI, nty = (jm + TJ - 1) / TJ, nks = (km + RT_KSEG - 1) / RT_KSEG;
+  const int ntx = (im + TI - 1) / TI, nty = (jm + TJ - 1) / TJ, nks = (km + kseg - 1) / kseg;
   int item = t.base;
   const int n = item / (ntx * nty * nks);
   item -= n * (ntx * nty * nks);
@@ -66,7 +68,7 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_tile(Par p, in
   item -= ks_i * (ntx * nty);
   const int ty_i = item / ntx, tx_i = item - ty_i * ntx;
   const int i0 = 1 + tx_i * TI, j0 = 1 + ty_i * TJ;
-  const int ks = 1 + ks_i * RT_KSEG, ke = min(km, ks + RT_KSEG - 1);
+  const int ks = 1 + ks_i * kseg, ke = min(km, ks + kseg - 1);
   const ll n3 = n3of(b);
   const T* qb = q + b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n;
   double* rb = res + b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n;
@@ -234,7 +236,7 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_tile(Par p, in
 //       barrier) and the cell sums them in the reference order.
 template <typename T, int TI, int TJ, int MINW>
 __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_sva(Par p, int nl, const Blk* __restrict__ blks,
-                                                                const Tile* __restrict__ tiles,
+                                                                const Tile* __restrict__ tiles, int kseg,
                                                                 const T* __restrict__ q, const T* __restrict__ si,
                                                                 const T* __restrict__ sj, const T* __restrict__ sk,
                                                                 double* __restrict__ res,
@@ -254,7 +256,7 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_sva(Par p, int
   const Blk b = blks[t.block];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int im = b.imax - 1, jm = b.jmax - 1, km = b.kmax - 1;
-  const int ntx = (im + TI - 1) / TI, nty = (jm + TJ - 1) / TJ, nks = (km + RT_KSEG - 1) / RT_KSEG;
+  const int ntx = (im + TI - 1) / TI, nty = (jm + TJ - 1) / TJ, nks = (km + kseg - 1) / kseg;
   int item = t.base;
   const int n = item / (ntx * nty * nks);
   item -= n * (ntx * nty * nks);
@@ -262,7 +264,7 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_sva(Par p, int
   item -= ks_i * (ntx * nty);
   const int ty_i = item / ntx, tx_i = item - ty_i * ntx;
   const int i0 = 1 + tx_i * TI, j0 = 1 + ty_i * TJ;
-  const int ks = 1 + ks_i * RT_KSEG, ke = min(km, ks + RT_KSEG - 1);
+  const int ks = 1 + ks_i * kseg, ke = min(km, ks + kseg - 1);
   const ll n3 = n3of(b);
   const T* qb = q + b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n;
   double* rb = res + b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n;
@@ -450,14 +452,14 @@ template <typename T, int TJ, int ILIM, int FO, int EF, int KW, int MINW = 1, in
 static void launch_tile(Solve& s, Level& L, int ntile, const Tile* tiles, const T* q, const T* si, const T* sj,
                         const T* sk, double* res) {
   hipLaunchKernelGGL((k_residual_tile<T, TI, TJ, ILIM, FO, EF, KW, MINW>), dim3(ntile), dim3(32 * (TJ + 1)), 0,
-                     s.stream, s.par, L.nl, L.dblk, tiles, q, si, sj, sk, res, L.sbc, L.sbc_doff);
+                     s.stream, s.par, L.nl, L.dblk, tiles, L.kseg, q, si, sj, sk, res, L.sbc, L.sbc_doff);
 }
 
 template <typename T, int TJ, int MINW = 1, int TI = 31>
 static void launch_sva(Solve& s, Level& L, int ntile, const Tile* tiles, const T* q, const T* si, const T* sj,
                        const T* sk, double* res) {
   hipLaunchKernelGGL((k_residual_sva<T, TI, TJ, MINW>), dim3(ntile), dim3(32 * (TJ + 1)), 0, s.stream, s.par, L.nl,
-                     L.dblk, tiles, q, si, sj, sk, res, L.sbc, L.sbc_doff);
+                     L.dblk, tiles, L.kseg, q, si, sj, sk, res, L.sbc, L.sbc_doff);
 }
 
 // The instances built: van Albada (the default limiter) specialised, every
@@ -527,9 +529,43 @@ hipError_t launch_residual_tile_contracted(Solve& s, Level& L, int variant, cons
 #else
 // Work items of one block for a TI x TJ tile table: (i tiles) x (j tiles) x
 // (k segments) x snapshots, i tiles fastest.
-ll residual_tile_items(int TI, int TJ, int imax, int jmax, int kmax, int nsnap) {
+ll residual_tile_items(int TI, int TJ, int kseg, int imax, int jmax, int kmax, int nsnap) {
   const ll im = imax - 1, jm = jmax - 1, km = kmax - 1;
-  return (ll)nsnap * ((im + TI - 1) / TI) * ((jm + TJ - 1) / TJ) * ((km + RT_KSEG - 1) / RT_KSEG);
+  return (ll)nsnap * ((im + TI - 1) / TI) * ((jm + TJ - 1) / TJ) * ((km + kseg - 1) / kseg);
+}
+
+// k-planes per work-group of a level's residual tiles.  A work-group's planes
+// run one after the other, so a level whose tiles do not fill the chip is cut
+// into short segments; each segment costs about half a plane more than its
+// planes (its first k-face and column loads).  The estimate of a launch: one
+// plane of a work-group alone on its CU takes 8 us (a chain of divisions and
+// barriers), a CU with enough work-groups finishes one plane per 5.7 us, and
+// the last work-groups to start add most of a chain.  The shortest estimate
+// wins, the longer segments where two are equal.  Measured (us, 32-plane
+// segments -> this rule): one 17^3-node block 109 -> 14, the 193 x 49 x 9
+// O-grid 63 -> 21, 97 x 49 x 49 nodes 234 -> 36, 48 uneven blocks 1382 -> 1270
+// on level 1 and 284 -> 146 on level 2; over 17 levels of ten grids the
+// pick is within 5% of the best of 1, 2, 3, 4, 6, 8, 12, 16, 32.
+int residual_kseg(const std::vector<Blk>& blks, int nsnap) {
+  int best = RT_KSEG;
+  double tbest = 0;
+  for (int kseg = RT_KSEG; kseg >= 1; kseg--) {
+    double planes = 0;   // planes of all work-groups, half a plane more for each
+    int longest = 1;
+    for (const Blk& b : blks) {
+      const double tiles = (double)residual_tile_items(32, 7, b.kmax, b.imax, b.jmax, b.kmax, nsnap);
+      const int km = b.kmax - 1;
+      planes += tiles * (km + 0.5 * ((km + kseg - 1) / kseg));
+      longest = std::max(longest, std::min(kseg, km));
+    }
+    const double chain = longest + 0.5;
+    const double t = std::max(8.0 * chain, 5.7 * planes / 256 + 0.8 * 8.0 * chain);
+    if (tbest == 0 || t < tbest) {
+      tbest = t;
+      best = kseg;
+    }
+  }
+  return best;
 }
 
 hipError_t launch_residual_tile(Solve& s, Level& L, int variant, const double* q, const double* si,

@@ -27,8 +27,8 @@ namespace cosahip {
 
 template <typename T, int NV, bool VIS, int TI, int TJ, int ILIM, int FO, int EF>
 __global__ void __launch_bounds__(32 * (TJ + 1)) k_residual_tile_v(
-    Par p, int nl, const Blk* __restrict__ blks, const Tile* __restrict__ tiles, const T* __restrict__ q,
-    const T* __restrict__ si, const T* __restrict__ sj, const T* __restrict__ sk, double* __restrict__ res,
+    Par p, int nl, const Blk* __restrict__ blks, const Tile* __restrict__ tiles, int kseg,
+    const T* __restrict__ q, const T* __restrict__ si, const T* __restrict__ sj, const T* __restrict__ sk, double* __restrict__ res,
     const unsigned char* __restrict__ sbc, const ll* __restrict__ sbcoff, const double* __restrict__ h0tab,
     const T* __restrict__ vf, ll vslot) {
   constexpr int NT = 32 * (TJ + 1), PW = TI + 4, PH = TJ + 4;
@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(32 * (TJ + 1)) k_residual_tile_v(
   const Blk b = blks[t.block];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int im = b.imax - 1, jm = b.jmax - 1, km = b.kmax - 1;
-  const int ntx = (im + TI - 1) / TI, nty = (jm + TJ - 1) / TJ, nks = (km + RT_KSEG - 1) / RT_KSEG;
+  const int ntx = (im + TI - 1) / TI, nty = (jm + TJ - 1) / TJ, nks = (km + kseg - 1) / kseg;
   int item = t.base;
   const int n = item / (ntx * nty * nks);
   item -= n * (ntx * nty * nks);
@@ -48,7 +48,7 @@ __global__ void __launch_bounds__(32 * (TJ + 1)) k_residual_tile_v(
   item -= ks_i * (ntx * nty);
   const int ty_i = item / ntx, tx_i = item - ty_i * ntx;
   const int i0 = 1 + tx_i * TI, j0 = 1 + ty_i * TJ;
-  const int ks = 1 + ks_i * RT_KSEG, ke = min(km, ks + RT_KSEG - 1);
+  const int ks = 1 + ks_i * kseg, ke = min(km, ks + kseg - 1);
   const ll n3 = n3of(b);
   const T* qb = q + b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n;
   double* rb = res + b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n;
@@ -201,7 +201,7 @@ template <typename T, int NV, bool VIS, int ILIM, int FO, int EF>
 static void launch_v(Solve& s, Level& L, const T* q, const T* si, const T* sj, const T* sk, double* res,
                      const T* vf, ll vslot) {
   hipLaunchKernelGGL((k_residual_tile_v<T, NV, VIS, 32, 7, ILIM, FO, EF>), dim3(L.ntile[TK_T32]), dim3(256), 0,
-                     s.stream, s.par, L.nl, L.dblk, L.tile[TK_T32], q, si, sj, sk, res, L.sbc, L.sbc_doff, L.h0tab,
+                     s.stream, s.par, L.nl, L.dblk, L.tile[TK_T32], L.kseg, q, si, sj, sk, res, L.sbc, L.sbc_doff, L.h0tab,
                      vf, vslot);
 }
 
