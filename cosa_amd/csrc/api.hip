@@ -266,7 +266,7 @@ int cosahip_create(const cosahip_config* cfg, int device, cosahip_solve** out) {
   const char* gk = getenv("COSAHIP_GRAPH");
   s->use_graph = !(gk && strcmp(gk, "0") == 0);
   const char* ck = getenv("COSAHIP_CIRS_I");
-  s->cirs_i_mode = !ck ? 0 : strcmp(ck, "lds") == 0 ? 1 : strcmp(ck, "iv") == 0 ? 2 : strcmp(ck, "line") == 0 ? 3 : 0;
+  s->cirs_i_mode = !ck ? 0 : strcmp(ck, "lds") == 0 || strcmp(ck, "iv") == 0 ? 2 : strcmp(ck, "line") == 0 ? 3 : 0;
   const char* lk = getenv("COSAHIP_CIRS_IL_LDS");
   if (lk) s->il_lds = std::min(65536, std::max(4096, atoi(lk)));
   const char* vk = getenv("COSAHIP_VISCOUS");
@@ -274,7 +274,8 @@ int cosahip_create(const cosahip_config* cfg, int device, cosahip_solve** out) {
   s->viscous_faces = !(vk && (strcmp(vk, "march") == 0 || strcmp(vk, "fused") == 0));
   s->viscous_tile = !(vk && (strcmp(vk, "march") == 0 || strcmp(vk, "fused") == 0 || strcmp(vk, "faces") == 0));
   const char* jk = getenv("COSAHIP_CIRS_JK");
-  s->cirs_jk_chunk = !jk ? 4 : strcmp(jk, "plain") == 0 ? 0 : strcmp(jk, "chunk8") == 0 ? 8 : 4;
+  s->cirs_jk_mode = !jk ? 2 : strcmp(jk, "plain") == 0 ? 0 : strncmp(jk, "chunk", 5) == 0 ? 1 : 2;
+  s->cirs_jk_chunk = jk && strcmp(jk, "chunk8") == 0 ? 8 : 4;
   if (device >= 0) {
     if (hipSetDevice(device) != hipSuccess) {
       delete s;
@@ -364,25 +365,49 @@ static void add_tiles(std::vector<Tile>& v, int block, ll items, int per) {
   for (ll b0 = 0; b0 < items; b0 += per) v.push_back(Tile{block, (int)b0});
 }
 
-// k_cirs_il (CIRS i-sweep, constant coefficient of irsop 1): how many whole
-// lines of all npde variables one work-group keeps in LDS, within
-// s->il_lds bytes (two tables, lines, per-row offsets; default 24 KB, so that
-// six work-groups share a CU), raised to what one line needs for long lines
-// (at most 64 KB).
-
+// k_cirs_il (CIRS i-sweep): how many whole lines of all variables (with
+// variable coefficients their coefficients and multipliers too) one
+// work-group keeps in LDS, within s->il_lds bytes (default 40 KB, so that three
+// work-groups share a CU), raised to what one line needs for long lines (at
+// most half a CU's LDS).  A level of few lines is spread over two work-groups
+// per CU rather than kept in full ones.
 static void plan_cirs_il(Solve* s, Level& L) {
   L.il_lpw = 0;
   L.il_stride = 0;
-  if (s->par.irsop != 1 || !L.nblocks) return;
+  if (s->par.irsop < 1 || !L.nblocks) return;
   int lmax = 1;
-  for (const Blk& B : L.hblk) lmax = std::max(lmax, B.imax - 1);
-  const int S = lmax | 1;
-  const int nv = s->par.npde;
-  const int budget = std::max(s->il_lds, std::min(65536, 16 * S + nv * (8 * S + 16)));
-  const int lpw = std::min((budget - 16 * S) / (nv * (8 * S + 16)), 256 / nv);
-  if (lpw < 1) return;
-  L.il_lpw = lpw;
-  L.il_stride = S;
+  ll lines = 0;
+  for (const Blk& B : L.hblk) {
+    lmax = std::max(lmax, B.imax - 1);
+    lines += (ll)s->par.nsnap * (B.jmax - 1) * (B.kmax - 1);
+  }
+  const ll S = lmax | 1, tab = s->par.irsop == 1 ? 16 * S + 8 : 0, row = 8 * S * cirs_strip_per(s->par);
+  if (tab + row > 79000) return;
+  ll lpw = std::max<ll>(1, (s->il_lds - tab) / row);
+  lpw = std::min(lpw, std::min<ll>(256 / s->par.npde, (lines + 511) / 512));
+  L.il_lpw = (int)lpw;
+  L.il_stride = (int)S;
+  L.il_lds = (size_t)(tab + lpw * row);
+}
+
+// k_cirs_strip: LDS bytes of a work-group per direction, the largest over the
+// blocks; 0 (the line kernels instead) when some block's line does not fit.
+static void plan_cirs_strip(Solve* s, Level& L) {
+  const int per = cirs_strip_per(s->par), nv = s->par.npde;
+  for (int d = 0; d < 2; d++) {
+    L.strip_lds[d] = 0;
+    if (s->par.irsop < 1 || s->cirs_jk_mode != 2) continue;
+    for (const Blk& b : L.hblk) {
+      const int n = (d == 0 ? b.jmax : b.kmax) - 1, w = cirs_strip_w(n, b.imax - 1, per);
+      if (!w || n >= JK_RT) {
+        L.strip_lds[d] = 0;
+        break;
+      }
+      const size_t bytes = sizeof(double) * ((size_t)nv * cirs_strip_vs(n, w) +
+                                             (s->par.irsop == 1 ? 2 * (size_t)n + 1 : (size_t)(per - nv) * n * w));
+      L.strip_lds[d] = std::max(L.strip_lds[d], bytes);
+    }
+  }
 }
 
 // Per block, the Thomas multipliers r(a) = c(a) / (b(a) - r(a-1) a(a)) of
@@ -395,7 +420,7 @@ static void plan_cirs_il(Solve* s, Level& L) {
 static int upload_cirs_il_table(Solve* s, Level& L) {
   if (L.il_rtab) (void)hipFree(L.il_rtab);
   L.il_rtab = nullptr;
-  if (!L.il_lpw) return COSAHIP_OK;
+  if (!L.il_lpw || s->par.irsop != 1) return COSAHIP_OK;
   const double epsc = 0.25 * (s->par.rat * s->par.rat - 1.0);
   const size_t S = L.il_stride;
   std::vector<double> tab((size_t)L.nblocks * 2 * S, 0.0);
@@ -450,6 +475,7 @@ static int build_tables(Solve* s, Level& L, const Level* Lc) {
   for (int k = 0; k < TK_NKIND; k++) L.htile[k].clear();
   plan_cirs_il(s, L);
   L.kseg = residual_kseg(L.hblk, ns);
+  plan_cirs_strip(s, L);
   for (int b = 0; b < L.nblocks; b++) {
     const Blk& B = L.hblk[b];
     const ll im = B.imax - 1, jm = B.jmax - 1, km = B.kmax - 1;
@@ -460,10 +486,14 @@ static int build_tables(Solve* s, Level& L, const Level* Lc) {
     add_tiles(L.htile[TK_LINES_K], b, ns * im * jm, TS);
     add_tiles(L.htile[TK_SEGS_J], b, ns * im * km * ((jm + MSEG - 1) / MSEG), TS);
     add_tiles(L.htile[TK_SEGS_K], b, ns * im * jm * ((km + MSEG - 1) / MSEG), TS);
-    add_tiles(L.htile[TK_LINES_I], b, ns * jm * km, 64);
     add_tiles(L.htile[TK_LINES_I_T], b, ns * jm * km, TS);
     add_tiles(L.htile[TK_LINES_IV], b, ns * jm * km, 256 / s->par.npde);
     if (L.il_lpw) add_tiles(L.htile[TK_LINES_IL], b, ns * jm * km, L.il_lpw);
+    for (int d = 0; d < 2; d++)
+      if (L.strip_lds[d]) {
+        const int w = cirs_strip_w((int)(d == 0 ? jm : km), (int)im, cirs_strip_per(s->par));
+        add_tiles(L.htile[d == 0 ? TK_STRIP_J : TK_STRIP_K], b, ns * ((im + w - 1) / w) * (d == 0 ? km : jm), 1);
+      }
     if (s->par.viscous) {
       add_tiles(L.htile[TK_FACES_I], b, ns * (im + 1) * jm * km, TS);
       add_tiles(L.htile[TK_FACES_J], b, ns * im * (jm + 1) * km, TS);
@@ -2255,14 +2285,12 @@ extern "C" int cosahip_autotune(cosahip_solve* h, int reps, int32_t* choice) {
     std::swap(L.f[COSAHIP_RES], L.work1);
     float t[4] = {0, 0, 0, 0};
     const int last = L.ntile[TK_LINES_IL] ? 3 : 2;
-    for (int mode = 1; mode <= last && rc == COSAHIP_OK; mode++) {
+    for (int mode = 2; mode <= last && rc == COSAHIP_OK; mode++) {
       L.cirs_mode = mode;
       rc = timed([&]() { return launch_cirs(*s, L); }, t[mode]);
     }
     std::swap(L.f[COSAHIP_RES], L.work1);
-    L.cirs_mode = 1;
-    for (int mode = 2; mode <= last; mode++)
-      if (t[mode] < t[L.cirs_mode]) L.cirs_mode = mode;
+    L.cirs_mode = last == 3 && t[3] < t[2] ? 3 : 2;
     if (choice) choice[nl - 1] = L.cirs_mode;
   }
   // inviscid residual kernel per level: timed into work1 (q is only read)

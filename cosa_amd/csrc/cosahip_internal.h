@@ -86,7 +86,6 @@ enum TileKind {
   TK_ROWS_I,      // i-direction flux rows: (jmax-1)(kmax-1) rows x segments
   TK_LINES_J,     // (imax-1)(kmax-1) lines along j
   TK_LINES_K,     // (imax-1)(jmax-1) lines along k
-  TK_LINES_I,     // (jmax-1)(kmax-1) lines along i, 64 per tile
   TK_CELLS_P1,    // 0..imax x 0..jmax x 0..kmax
   TK_COARSE,      // cells of the next coarser level, per block (restriction)
   TK_PROL,        // 2x2x2 prolongation groups 0..imax-1 step 2, per block
@@ -102,9 +101,29 @@ enum TileKind {
   TK_FACES_K,     // k faces (imax-1) x (jmax-1) x kmax
   TK_FUSED15,     // residual tiles of 31 x 15 cells x kseg-plane k segments (k_residual_tile, TJ = 15)
   TK_SHELL,       // the halo shell of 0..imax x 0..jmax x 0..kmax (the box without the interior cells)
+  TK_STRIP_J,     // strips of cirs_strip_w lines along j (W cells along i x the whole j-line, all variables)
+  TK_STRIP_K,     // the same along k
   TK_T32,         // residual tiles of 32 x 7 cells x kseg-plane k segments (RESID_TILE32_W4, RESID_SVA32)
   TK_NKIND
 };
+
+// k_cirs_strip: lines (cells along i) of one work-group for lines of L cells
+// in a block im cells wide, per = doubles of LDS per cell of a line.  A power
+// of two; whole lines stay within 40 KB, so that three or four work-groups
+// share a CU, as long as that leaves 8 (a 64-byte run in memory); longer
+// lines keep 8 up to the LDS of half a CU and then 4.  0: the line does not fit.
+__host__ __device__ inline int cirs_strip_w(int L, int im, int per) {
+  int w = 32;   // 32 x 7 variables fit the threads of a work-group
+  while (w > 8 && ((ll)w * L * per * 8 > 40960 || w >= 2 * im)) w >>= 1;
+  if ((ll)w * L * per * 8 > 79000) w = 4;
+  return (ll)w * L * per * 8 > 79000 ? 0 : w;
+}
+// doubles of LDS per cell: the variables and, with variable coefficients, the
+// coefficient and multiplier of the mean flow and of k-omega
+inline int cirs_strip_per(const Par& p) { return p.npde + (p.irsop == 1 ? 0 : p.npde > 5 ? 4 : 2); }
+// LDS stride of one variable's strip in doubles: the variables' lanes of a
+// half-wave fall into different banks
+__host__ __device__ inline int cirs_strip_vs(int L, int w) { return w < 32 ? ((L * w + 31) & ~31) + w : L * w; }
 
 // inviscid residual kernels (the same bits; chosen per level by
 // cosahip_autotune or COSAHIP_RESIDUAL at create time)
@@ -192,11 +211,13 @@ struct Level {
   double* dq = nullptr;       // HB term (qhb) and scratch
   double* work1 = nullptr;    // copy of res for the HB norm
   double* dqc = nullptr;      // SST: (P3, 9, nsnap) cell-centre velocity differences of the stage
-  int cirs_mode = 0;          // CIRS i-sweep picked by cosahip_autotune: 0 none, 1 lds, 2 iv, 3 line
+  int cirs_mode = 0;          // CIRS i-sweep picked by cosahip_autotune: 0 none, 2 iv, 3 line
   int resid_mode = RESID_SVA32;   // inviscid residual kernel (ResidVariant)
   int kseg = 1;               // k-planes per work-group of the residual tiles (residual_kseg)
   int il_lpw = 0;             // k_cirs_il: lines per work-group (0: lines too long for its LDS budget)
   int il_stride = 0;          // k_cirs_il: odd LDS row stride >= the longest i-line of the level
+  size_t il_lds = 0;          // k_cirs_il: LDS bytes per work-group
+  size_t strip_lds[2] = {};   // k_cirs_strip, j and k lines: LDS bytes per work-group (0: some line does not fit)
   double* il_rtab = nullptr;  // k_cirs_il: multipliers and reciprocal divisors, 2 il_stride per block
   double* jk_rtab[2] = {};    // k_cirs_jk (irsop 1), j and k lines: r(a) and 1/d(a), a = 1..L, 2 (JK_RT) per block
   double* cirs_r = nullptr;   // Thomas multipliers r(j), one per cell
@@ -300,14 +321,15 @@ struct Solve {
   bool fuse_viscous = false;
   bool viscous_faces = true;
   bool viscous_tile = true;
-  // CIRS i-sweep: one thread per (line, variable) on levels with fewer than
-  // CIRS_IV_MAX_LINES lines along i, one thread per line with LDS-staged
-  // chunks on larger ones; COSAHIP_CIRS_I=lds|iv at create time forces one
-  int cirs_i_mode = 0;   // 0 auto, 1 lds, 2 iv, 3 line
-  int il_lds = 24576;    // LDS bytes per work-group of the line-resident CIRS i-sweep
-  // CIRS j/k sweeps of irsop 1: the forward pass kept in chunks of 4 cells
-  // (k_cirs_jkc, the default; measured fastest) or 8 (COSAHIP_CIRS_JK=chunk8
-  // at create time), or stored whole (0, COSAHIP_CIRS_JK=plain)
+  // CIRS i-sweep: whole lines resident in LDS where they fit, else one thread
+  // per (line, variable); COSAHIP_CIRS_I=line|iv at create time forces one
+  int cirs_i_mode = 0;   // 0 auto, 2 iv, 3 line
+  int il_lds = 40960;    // LDS bytes per work-group of the line-resident CIRS i-sweep
+  // CIRS j/k sweeps: 2 whole lines resident in LDS (k_cirs_strip, default)
+  // where they fit, 1 for irsop 1 the forward pass kept in chunks of 4 or 8
+  // cells (k_cirs_jkc; COSAHIP_CIRS_JK=chunk4|chunk8 at create time), 0 the
+  // forward pass stored whole (k_cirs_jk; COSAHIP_CIRS_JK=plain)
+  int cirs_jk_mode = 2;
   int cirs_jk_chunk = 4;
   // residual precision: 0 FP64, 1 FP32 residual / FP64 state, 2 FP32 until
   // the level-1 density residual rms falls below prec_tail_rms, FP64 after,
@@ -356,6 +378,5 @@ constexpr int TS = 256;        // items per tile, 1-D kernels
 constexpr int JK_RT = 1025;    // per-block stride of the j/k CIRS tables (lines up to 1024 cells)
 constexpr int ROWSEG = 63;     // cells per i-row segment (64 faces)
 constexpr int MSEG = 16;       // cells per segment of a j / k line march
-constexpr ll CIRS_IV_MAX_LINES = 262144;   // i-lines (x snapshots) of a level below which k_cirs_iv is used
 
 }  // namespace cosahip

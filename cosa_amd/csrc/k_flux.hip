@@ -565,154 +565,7 @@ __global__ void __launch_bounds__(256) k_lambda_deltat(Par p, const Blk* __restr
 // res by the time step (dtvol, or dtvolt for k, omega), the k sweep divides
 // it back; epsc is the constant coefficient of irsop = 1.
 
-// CIRS along i, where each line is contiguous in memory: one wavefront per
-// 64 lines.  Chunks of CI cells of every line (five variables, dtvol and the
-// coefficients) are staged through LDS with coalesced loads and stores; the
-// per-line Thomas recurrence then runs from LDS with the same arithmetic as
-// k_cirs_jk (forward pass r, t; backward pass x).  This is always the first
-// sweep: res is scaled by dtvol on load.
-constexpr int CI = 8;     // cells per chunk
-constexpr int LPAD = 65;  // padded line stride in LDS (conflict-free lane access)
-
-template <int NV>
-__global__ void __launch_bounds__(64) k_cirs_i(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
-                                               double* __restrict__ res, const double* __restrict__ dtvol,
-                                               const double* __restrict__ beta, double* __restrict__ rsc, int v0,
-                                               double epsc) {
-  __shared__ double xs[NV][CI][LPAD];
-  __shared__ double rsh[CI][LPAD];
-  __shared__ double dsh[CI][LPAD];
-  __shared__ double bsh[CI][LPAD];
-  const Tile t = tiles[blockIdx.x];
-  const Blk b = blks[t.block];
-  const int lane = threadIdx.x;
-  const int im = b.imax - 1, jm = b.jmax - 1, km = b.kmax - 1;
-  const int nlines = jm * km;
-  const int total = nlines * p.nsnap;
-  const int nl_here = min(64, total - t.base);
-  const int L = im;
-  const ll n3 = n3of(b), n1 = n1of(b);
-  const bool cb_const = p.irsop == 1;
-  // load slots: position ii = lane % CI of the chunk for lines lane/CI + 8 r
-  const int ii_ld = lane % CI;
-  ll off3[8], offr[8], off1[8];
-  bool ok[8];
-#pragma unroll
-  for (int r = 0; r < 8; r++) {
-    const int ln = lane / CI + 8 * r;
-    ok[r] = ln < nl_here;
-    const int gl = t.base + (ok[r] ? ln : 0);
-    const int n = gl / nlines, rem = gl - (gl / nlines) * nlines;
-    const int j = rem % jm + 1, k = rem / jm + 1;
-    off3[r] = b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n + n3 * v0 + i3(b, 0, j, k);
-    offr[r] = b.o3 * p.nsnap + n3 * (ll)n + i3(b, 0, j, k);
-    off1[r] = b.o1 * p.nsnap + n1 * (ll)n + i1(b, 0, j, k);
-  }
-  const bool active = lane < nl_here;
-  double tp[NV];
-  double rp = 0.0;
-  const int nchunk = (L + CI - 1) / CI;
-  // forward elimination
-  for (int c = 0; c < nchunk; c++) {
-    const int i0 = 1 + c * CI;
-    const int cnt = min(CI, L - i0 + 1);
-    if (ii_ld < cnt) {
-#pragma unroll
-      for (int r = 0; r < 8; r++) {
-        if (!ok[r]) continue;
-        const int ln = lane / CI + 8 * r;
-        const int i = i0 + ii_ld;
-#pragma unroll
-        for (int v = 0; v < NV; v++) xs[v][ii_ld][ln] = res[off3[r] + n3 * v + i];
-        dsh[ii_ld][ln] = dtvol[off1[r] + i];
-        if (!cb_const) bsh[ii_ld][ln] = beta[off1[r] + i];
-      }
-    }
-    __syncthreads();
-    if (active) {
-      for (int ii = 0; ii < cnt; ii++) {
-        const int a = i0 + ii;
-        const double eps = cb_const ? epsc : bsh[ii][lane];
-        const double ca = a == 1 ? 0.0 : -eps;
-        const double cb = 1 + 2 * eps;
-        const double cc = a == L ? 0.0 : -eps;
-        const double dtv = dsh[ii][lane];
-        double r;
-        if (a == 1) {
-          r = cc / cb;
-#pragma unroll
-          for (int v = 0; v < NV; v++) tp[v] = (xs[v][ii][lane] * dtv) / cb;
-        } else {
-          r = cc / (cb - rp * ca);
-#pragma unroll
-          for (int v = 0; v < NV; v++) tp[v] = (xs[v][ii][lane] * dtv - tp[v] * ca) / (cb - rp * ca);
-        }
-        rp = r;
-        rsh[ii][lane] = r;
-#pragma unroll
-        for (int v = 0; v < NV; v++) xs[v][ii][lane] = tp[v];
-      }
-    }
-    __syncthreads();
-    if (ii_ld < cnt) {
-#pragma unroll
-      for (int r = 0; r < 8; r++) {
-        if (!ok[r]) continue;
-        const int ln = lane / CI + 8 * r;
-        const int i = i0 + ii_ld;
-#pragma unroll
-        for (int v = 0; v < NV; v++) res[off3[r] + n3 * v + i] = xs[v][ii_ld][ln];
-        rsc[offr[r] + i] = rsh[ii_ld][ln];
-      }
-    }
-    __syncthreads();
-  }
-  // back substitution
-  double xn[NV];
-  for (int c = nchunk - 1; c >= 0; c--) {
-    const int i0 = 1 + c * CI;
-    const int cnt = min(CI, L - i0 + 1);
-    if (ii_ld < cnt) {
-#pragma unroll
-      for (int r = 0; r < 8; r++) {
-        if (!ok[r]) continue;
-        const int ln = lane / CI + 8 * r;
-        const int i = i0 + ii_ld;
-#pragma unroll
-        for (int v = 0; v < NV; v++) xs[v][ii_ld][ln] = res[off3[r] + n3 * v + i];
-        rsh[ii_ld][ln] = rsc[offr[r] + i];
-      }
-    }
-    __syncthreads();
-    if (active) {
-      for (int ii = cnt - 1; ii >= 0; ii--) {
-        const int a = i0 + ii;
-        if (a == L) {
-#pragma unroll
-          for (int v = 0; v < NV; v++) xn[v] = xs[v][ii][lane];
-        } else {
-          const double r = rsh[ii][lane];
-#pragma unroll
-          for (int v = 0; v < NV; v++) xn[v] = xs[v][ii][lane] - xn[v] * r;
-        }
-#pragma unroll
-        for (int v = 0; v < NV; v++) xs[v][ii][lane] = xn[v];
-      }
-    }
-    __syncthreads();
-    if (ii_ld < cnt) {
-#pragma unroll
-      for (int r = 0; r < 8; r++) {
-        if (!ok[r]) continue;
-        const int ln = lane / CI + 8 * r;
-        const int i = i0 + ii_ld;
-#pragma unroll
-        for (int v = 0; v < NV; v++) res[off3[r] + n3 * v + i] = xs[v][ii_ld][ln];
-      }
-    }
-    __syncthreads();
-  }
-}
+constexpr int CI = 8;     // cells per register chunk of k_cirs_iv
 
 // CIRS multipliers of the constant coefficient (irsop 1) in LDS: tridi's
 // r(a) = c(a) / (b(a) - r(a-1) a(a)) depend only on the position along the
@@ -1149,6 +1002,245 @@ __global__ void __launch_bounds__(256) k_cirs_jkc(Par p, const Blk* __restrict__
   }
 }
 
+// The recurrence of one line resident in LDS, cell a = 0 .. L - 1 at x[a W].
+// Runs of eight cells (then four, two, one) are loaded to registers together
+// before the chain uses them, so the chain waits for the LDS once per run: a
+// bounds test per cell made it four times as long, loading the next run ahead
+// of the chain nothing (its registers cost waves).  The ends need no case of
+// their own: t(-1) = -0 leaves x(0) as it is (ca < 0), and r(L-1) = 0 does the
+// same for the back substitution.
+//
+// Forward, constant coefficient: t(a) = (x(a) - t(a-1) ca) / d(a), the quotient
+// from the table's reciprocal divisor with Markstein's correction as in
+// k_cirs_jk; an exact zero n keeps its sign without a test: q d - n is +0
+// there, and -(+0) y + q is q (d, y > 0).  r(a - 1) is read at r[a], d(a)
+// formed from it.
+__device__ __forceinline__ double table_quotient(double n, double d, double y) {
+  const double q = n * y;
+  return fma(-fma(q, d, -n), y, q);
+}
+template <int U>
+__device__ __forceinline__ double strip_forward_run(double* __restrict__ x, const double* __restrict__ r,
+                                                    const double* __restrict__ y, int a0, int W, double ca, double cb,
+                                                    double tp) {
+  double xv[U], dv[U], yv[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    xv[u] = x[(a0 + u) * W];
+    dv[u] = cb - r[a0 + u] * ca;
+    yv[u] = y[a0 + u];
+  }
+#pragma unroll
+  for (int u = 0; u < U; u++) xv[u] = tp = table_quotient(xv[u] - tp * ca, dv[u], yv[u]);
+#pragma unroll
+  for (int u = 0; u < U; u++) x[(a0 + u) * W] = xv[u];
+  return tp;
+}
+__device__ __forceinline__ void strip_forward(double* __restrict__ x, const double* __restrict__ r,
+                                              const double* __restrict__ y, int L, int W, double epsc) {
+  const double ca = -epsc, cb = 1 + 2 * epsc;
+  double tp = -0.0;
+  int a = 0;
+  for (; a + 8 <= L; a += 8) tp = strip_forward_run<8>(x, r, y, a, W, ca, cb, tp);
+  if (L & 4) tp = strip_forward_run<4>(x, r, y, a, W, ca, cb, tp);
+  if (L & 2) tp = strip_forward_run<2>(x, r, y, L & ~3, W, ca, cb, tp);
+  if (L & 1) strip_forward_run<1>(x, r, y, L - 1, W, ca, cb, tp);
+}
+// Forward, coefficients eps(a) at g[a W]; store: keep the multipliers r(a)
+// at r[a W] for every line of the group.  (At a = 0 tridi's a is 0, here
+// t(-1) = r(-1) = -0 take its place.)
+template <int U>
+__device__ __forceinline__ void strip_forward_v_run(double* __restrict__ x, const double* __restrict__ g,
+                                                    double* __restrict__ r, int a0, int L, int W, bool store,
+                                                    double& tp, double& rp) {
+  double xv[U], ev[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    xv[u] = x[(a0 + u) * W];
+    ev[u] = g[(a0 + u) * W];
+  }
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const double ca = -ev[u], cb = 1 + 2 * ev[u], cc = a0 + u == L - 1 ? 0.0 : -ev[u];
+    const double d = cb - rp * ca;
+    xv[u] = tp = (xv[u] - tp * ca) / d;
+    ev[u] = rp = cc / d;
+  }
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    x[(a0 + u) * W] = xv[u];
+    if (store) r[(a0 + u) * W] = ev[u];
+  }
+}
+__device__ __forceinline__ void strip_forward_v(double* __restrict__ x, const double* __restrict__ g,
+                                                double* __restrict__ r, int L, int W, bool store) {
+  double tp = -0.0, rp = -0.0;
+  int a = 0;
+  for (; a + 8 <= L; a += 8) strip_forward_v_run<8>(x, g, r, a, L, W, store, tp, rp);
+  if (L & 4) strip_forward_v_run<4>(x, g, r, a, L, W, store, tp, rp);
+  if (L & 2) strip_forward_v_run<2>(x, g, r, L & ~3, L, W, store, tp, rp);
+  if (L & 1) strip_forward_v_run<1>(x, g, r, L - 1, L, W, store, tp, rp);
+}
+// Back substitution x(a) = t(a) - x(a+1) r(a), r(a) at r[a RW].
+template <int U>
+__device__ __forceinline__ double strip_back_run(double* __restrict__ x, const double* __restrict__ r, int a1, int W,
+                                                 int RW, double xn) {
+  double xv[U], rv[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    xv[u] = x[(a1 - u) * W];
+    rv[u] = r[(a1 - u) * RW];
+  }
+#pragma unroll
+  for (int u = 0; u < U; u++) xv[u] = xn = xv[u] - xn * rv[u];
+#pragma unroll
+  for (int u = 0; u < U; u++) x[(a1 - u) * W] = xv[u];
+  return xn;
+}
+__device__ __forceinline__ void strip_back(double* __restrict__ x, const double* __restrict__ r, int L, int W, int RW) {
+  double xn = 0.0;
+  int a = L - 1;
+  for (; a >= 7; a -= 8) xn = strip_back_run<8>(x, r, a, W, RW, xn);
+  if (L & 4) xn = strip_back_run<4>(x, r, a, W, RW, xn);
+  if (L & 2) xn = strip_back_run<2>(x, r, (L & 3) - 1, W, RW, xn);
+  if (L & 1) strip_back_run<1>(x, r, 0, W, RW, xn);
+}
+
+// CIRS j / k sweep with whole lines resident in LDS: a work-group takes W
+// consecutive lines (cells along i, cirs_strip_w) of one block with all
+// variables.  The strip is read once in rows of W cells, one thread per (line,
+// variable) runs tridi's recurrence (src/cosa.f90:2418-2443) from LDS, and
+// the strip leaves once: as the smoothed residual, or through the RK update
+// and cons2prim (UPD as in k_cirs_jk).  Operations and order are those of
+// k_cirs_jk, so the bits are the same.  Memory bounds it: per cell one read
+// and one write of res (UPD: q written instead, qold and the time step read)
+// where the chunked sweep read res twice; a thread's recurrence waits on LDS
+// instead of HBM.  Level 1 of 48 uneven blocks (11.8 M cells): j 455 -> 329
+// us, k with the update 673 -> 505; 128 x 33 x 5 O-grids and SST j-lines with
+// variable coefficients 135 -> 24.  Narrower strips or 20 KB were no faster.
+// CC: the constant coefficient of irsop 1, multipliers r(a) and reciprocal
+// divisors from the block's table; else each thread forms r(a) from the
+// coefficients staged in LDS and the first thread of a group (mean flow,
+// k-omega) keeps it for the back substitution.
+template <int DIR, int NM, int NT, int UPD, bool CC>
+__global__ void __launch_bounds__(256) k_cirs_strip(Par p, const Blk* __restrict__ blks,
+                                                    const Tile* __restrict__ tiles, double* __restrict__ res,
+                                                    const double* __restrict__ dtvol,
+                                                    const double* __restrict__ dtvolt,
+                                                    const double* __restrict__ beta, const double* __restrict__ tbeta,
+                                                    int last, double epsc, CirsUpdate up,
+                                                    const double* __restrict__ jkt) {
+  constexpr int NV = NM + NT, NG = NT ? 2 : 1;
+  static_assert(UPD == 0 || (NM == 5 && NT == 0), "the fused update is built for the mean flow only");
+  extern __shared__ double sm[];
+  const Tile t = tiles[blockIdx.x];
+  const Blk b = blks[t.block];
+  const int im = b.imax - 1, jm = b.jmax - 1, km = b.kmax - 1;
+  const int L = DIR == 2 ? jm : km, T2 = DIR == 2 ? km : jm;
+  const int W = cirs_strip_w(L, im, NV + (CC ? 0 : 2 * NG)), VS = cirs_strip_vs(L, W);
+  const int nst = (im + W - 1) / W;
+  int item = t.base;
+  const int n = item / (nst * T2);
+  item -= n * (nst * T2);
+  const int t2 = item / nst + 1, i0 = (item - (t2 - 1) * nst) * W + 1;
+  const int tid = threadIdx.x;
+  // staging: thread (row ra, line w), rows RS apart
+  const int w = tid & (W - 1), ra = tid / W, RS = 256 / W;
+  const bool on = i0 + w <= im;
+  const ll n3 = n3of(b);
+  double* rb = res + b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n;
+  const ll sa = DIR == 2 ? (ll)(b.imax + 3) : (ll)(b.imax + 3) * (b.jmax + 3);   // cell stride along the line
+  const ll s1 = DIR == 2 ? (ll)(b.imax + 1) : (ll)(b.imax + 1) * (b.jmax + 1);   // the same in P1 arrays
+  const ll c3 = i3(b, i0 + w, DIR == 2 ? 1 : t2, DIR == 3 ? 1 : t2);             // cell a = 1 of line w
+  const ll c1 = b.o1 * p.nsnap + n1of(b) * (ll)n + i1(b, i0 + w, DIR == 2 ? 1 : t2, DIR == 3 ? 1 : t2);
+  double* xs = sm;
+  double* cf = sm + NV * VS;   // CC: r(-1) = -0, r(a), then 1/d(a); else per group eps(a), r(a) of every line
+  if (CC) {
+    const double* tb = jkt + 2 * (ll)JK_RT * t.block;
+    if (tid == 0) cf[0] = -0.0;
+    for (int a = tid; a < L; a += 256) {
+      cf[a + 1] = tb[a + 1];
+      cf[L + 1 + a] = tb[JK_RT + a + 1];
+    }
+  }
+  if (on) {
+#pragma unroll 4
+    for (int a = ra; a < L; a += RS) {
+#pragma unroll
+      for (int v = 0; v < NV; v++) xs[v * VS + a * W + w] = rb[c3 + a * sa + n3 * v];
+      if (!CC) {
+        cf[a * W + w] = beta[c1 + a * s1];
+        if (NT) cf[2 * L * W + a * W + w] = tbeta[c1 + a * s1];
+      }
+    }
+  }
+  __syncthreads();
+  // forward pass of line lw, variable lv
+  const int lv = tid / W, lw = w;
+  const bool line = lv < NV && i0 + lw <= im;
+  double* x = xs + lv * VS + lw;
+  double* g = cf + (!CC && NT && lv >= NM ? 2 * L * W : 0) + lw;   // the group's eps, then r
+  if (line) {
+    if (CC) strip_forward(x, cf, cf + L + 1, L, W, epsc);
+    else strip_forward_v(x, g, g + L * W, L, W, lv == 0 || (NT && lv == NM));
+  }
+  if (!CC) __syncthreads();
+  if (line) strip_back(x, CC ? cf + 1 : g + L * W, L, W, CC ? 1 : W);
+  __syncthreads();
+  if (!on) return;
+  const ll qo = rb - res;
+#pragma unroll 2
+  for (int a = ra; a < L; a += RS) {
+    const ll c = c3 + a * sa;
+    double xv[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) xv[v] = xs[v * VS + a * W + w];
+    if (UPD) {
+      const double dtv = dtvol[c1 + a * s1];
+      double qc[NM];
+#pragma unroll
+      for (int v = 0; v < NM; v++) {
+        const double rv = xv[v] / dtv;
+        qc[v] = up.qold[qo + c + n3 * v] - up.ar * rv * dtv;
+      }
+      double* qb = up.q + qo;
+      if (UPD == 2) {
+        const double rho = qc[0];
+        const double u_ = qc[1] / rho, vv = qc[2] / rho, w_ = qc[3] / rho;
+        const double pp = (p.gamma - 1) * (qc[4] - rho * (u_ * u_ + vv * vv + w_ * w_) / 2 - rho * 0.0);
+        qb[c] = rho;
+        qb[c + n3] = u_;
+        qb[c + 2 * n3] = vv;
+        qb[c + 3 * n3] = w_;
+        qb[c + 4 * n3] = pp;
+        if (up.q32) {
+          float* sb = up.q32 + qo;
+          sb[c] = (float)rho;
+          sb[c + n3] = (float)u_;
+          sb[c + 2 * n3] = (float)vv;
+          sb[c + 3 * n3] = (float)w_;
+          sb[c + 4 * n3] = (float)pp;
+        }
+      } else {
+#pragma unroll
+        for (int v = 0; v < NM; v++) qb[c + n3 * v] = qc[v];
+      }
+    } else if (last) {
+      const double dtv = dtvol[c1 + a * s1];
+#pragma unroll
+      for (int v = 0; v < NM; v++) rb[c + n3 * v] = xv[v] / dtv;
+      if (NT) {
+        const double dtvt = dtvolt[c1 + a * s1];
+#pragma unroll
+        for (int v = NM; v < NV; v++) rb[c + n3 * v] = xv[v] / dtvt;
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < NV; v++) rb[c + n3 * v] = xv[v];
+    }
+  }
+}
+
 // CIRS i-sweep with one thread per (line, variable): a 256-thread
 // workgroup takes 256 / NV lines, NV = npde variables each, so k and omega
 // are smoothed in the same launch as the mean flow.  Mean-flow variables
@@ -1157,8 +1249,8 @@ __global__ void __launch_bounds__(256) k_cirs_jkc(Par p, const Blk* __restrict__
 // line in chunks of CI cells whose loads are issued before the recurrence
 // consumes them.  The lanes of one line and group compute the same Thomas
 // multipliers and store them to the same address of rsc / rsct for the
-// back substitution.  Arithmetic as in k_cirs_i (tridi, src/cosa.f90:
-// 2418-2443).
+// back substitution.  Arithmetic of tridi (src/cosa.f90:2418-2443); for
+// lines too long for k_cirs_il.
 // With the constant coefficient of irsop 1 the multipliers depend only on
 // the position along the line: every line of a work-group (one block) has
 // the same, so they are computed once into LDS (RTAB_MAX cells at most)
@@ -1261,60 +1353,23 @@ __global__ void __launch_bounds__(256) k_cirs_iv(Par p, const Blk* __restrict__ 
   }
 }
 
-// One line of k_cirs_il: the forward and backward pass of the Thomas
-// recurrence over x (already scaled by the time step) in LDS.  Each forward
-// divisor d(a) = b - r(a-1) a(a) is known before the pass, so t(a) =
-// (x(a) - t(a-1) a(a)) / d(a) is formed from its reciprocal y(a) = RN(1/d)
-// as q = RN(n y), t = RN(q + (n - q d) y) with two fused multiply-adds:
-// with y correctly rounded, q faithful and no underflow (the residuals
-// here are far above the subnormal range), the correction gives the
-// correctly rounded quotient (Markstein's theorem; P. Markstein, IBM J. Res.
-// Dev. 34 (1990) 111-119), i.e. the same bits as n / d, with five
-// dependent operations instead of a full division.  An exact zero n is the
-// one case where the correction changes the sign (-0 + +0 rounds to +0):
-// there q = n y already is the signed zero n / d, so it is taken as is.
-// The restrict-qualified
-// arguments let the LDS reads of the next cells and table entries run ahead
-// of the stores of the recurrence.
-__device__ __forceinline__ void il_thomas(double* __restrict__ x, const double* __restrict__ r,
-                                          const double* __restrict__ y, int L, double ca, double cb) {
-  double tp;
-  {
-    const double n = x[0], q = n * y[0];
-    tp = n == 0.0 ? q : fma(fma(-q, cb, n), y[0], q);
-  }
-  x[0] = tp;
-  for (int a = 1; a < L; a++) {
-    const double d = cb - r[a - 1] * ca;
-    const double n = x[a] - tp * ca;
-    const double q = n * y[a];
-    tp = n == 0.0 ? q : fma(fma(-q, d, n), y[a], q);
-    x[a] = tp;
-  }
-  double xn = x[L - 1];
-  for (int a = L - 2; a >= 0; a--) {
-    xn = x[a] - xn * r[a];
-    x[a] = xn;
-  }
-}
-
-// CIRS i-sweep with whole lines resident in LDS (constant coefficient of
-// irsop 1): a work-group takes lpw lines of one block with all NV
-// variables.  The lines are read once with coalesced loads (row by row,
-// consecutive threads on consecutive cells), already multiplied by the time
-// step (dtvol, dtvolt for k and omega); one thread per (line, variable)
-// then runs il_thomas from LDS with the block's tables (multipliers r, the
-// values of fill_rtab, and the reciprocal divisors); the lines are written
-// back once.  Global traffic per cell is one read and one write of res plus
-// the time step, against two of each for the per-line sweeps.  Row stride S
-// is odd, so the lanes of the recurrence (S doubles apart) fall in distinct
-// LDS banks.  Results are those of k_cirs_iv (tridi, src/cosa.f90:
-// 2418-2443), bit for bit.
-template <int NV>
+// CIRS i-sweep with whole lines resident in LDS: a work-group takes lpw lines
+// of one block with all NV variables, one thread per (line, variable) runs
+// the recurrence of k_cirs_strip from LDS.  The lines are read once along i
+// (already multiplied by the time step, dtvol, or dtvolt for k and omega) and
+// written once, against two of each for the per-line sweep k_cirs_iv.  The
+// row stride S is odd, so the lanes of the recurrence (S doubles apart) fall
+// in distinct LDS banks.  CC: the constant coefficient of irsop 1 from the
+// block's table (multipliers and reciprocal divisors); else the coefficients
+// are staged with the line and the multipliers kept per line and group.
+// Results are those of k_cirs_iv (tridi, src/cosa.f90:2418-2443), bit for bit.
+template <int NM, int NT, bool CC>
 __global__ void __launch_bounds__(256) k_cirs_il(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                  double* __restrict__ res, const double* __restrict__ dtvol,
-                                                 const double* __restrict__ dtvolt, const double* __restrict__ tabs,
+                                                 const double* __restrict__ dtvolt, const double* __restrict__ beta,
+                                                 const double* __restrict__ tbeta, const double* __restrict__ tabs,
                                                  int lpw, int S, double epsc) {
+  constexpr int NV = NM + NT, NG = NT ? 2 : 1, NR = NV + (CC ? 0 : 2 * NG);   // LDS rows per line
   extern __shared__ double sm[];
   const Tile t = tiles[blockIdx.x];
   const Blk b = blks[t.block];
@@ -1322,39 +1377,63 @@ __global__ void __launch_bounds__(256) k_cirs_il(Par p, const Blk* __restrict__ 
   const int jm = b.jmax - 1, km = b.kmax - 1;
   const int nlines = jm * km;
   const int nl_here = min(lpw, nlines * p.nsnap - t.base);
-  const int nrow = NV * nl_here;
-  double* rt = sm;                              // r(a), a = 1..L at rt[a - 1]
-  double* yt = sm + S;                          // 1 / d(a) at yt[a - 1]
-  double* xs = sm + 2 * S;                      // row r = line * NV + variable
-  ll* base3 = reinterpret_cast<ll*>(xs + (ll)NV * lpw * S);
-  ll* base1 = base3 + NV * lpw;
   const ll n3 = n3of(b), n1 = n1of(b);
-  for (int r = threadIdx.x; r < nrow; r += blockDim.x) {
-    const int ln = r / NV, v = r - (r / NV) * NV;
+  double* rt = sm;                     // CC: r(-1) = -0, then r(a)
+  double* yt = sm + S + 1;             // CC: 1 / d(a)
+  double* xs = sm + (CC ? 2 * S + 1 : 0);  // row ln * NR + variable; else then eps, r of each group
+  if (CC) {
+    const double* tb = tabs + 2 * (ll)S * t.block;
+    if (threadIdx.x == 0) rt[0] = -0.0;
+    for (int a = threadIdx.x; a < L; a += 256) {
+      rt[a + 1] = tb[a];
+      yt[a] = tb[S + a];
+    }
+  }
+  // staging: TA threads along i, 256 / TA lines at a time
+  const int TA = L > 128 ? 256 : L > 64 ? 128 : L > 32 ? 64 : 32;
+  const int ta = threadIdx.x & (TA - 1);
+  auto base = [&](int ln, ll& o3, ll& o1) {
     const int gl = t.base + ln;
-    const int n = gl / nlines, rem = gl - (gl / nlines) * nlines;
+    const int n = gl / nlines, rem = gl - n * nlines;
     const int j = rem % jm + 1, k = rem / jm + 1;
-    base3[r] = b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n + n3 * v + i3(b, 0, j, k);
-    base1[r] = b.o1 * p.nsnap + n1 * (ll)n + i1(b, 0, j, k);
-  }
-  const double* tb = tabs + 2 * (ll)S * t.block;
-  for (int a = threadIdx.x; a < L; a += blockDim.x) {
-    rt[a] = tb[a];
-    yt[a] = tb[S + a];
+    o3 = b.o3 * p.npde * p.nsnap + n3 * (ll)p.npde * n + i3(b, 1, j, k);
+    o1 = b.o1 * p.nsnap + n1 * (ll)n + i1(b, 1, j, k);
+  };
+#pragma unroll 2
+  for (int ln = threadIdx.x / TA; ln < nl_here; ln += 256 / TA) {
+    ll o3, o1;
+    base(ln, o3, o1);
+    for (int a = ta; a < L; a += TA) {
+      const double dt = dtvol[o1 + a], dtt = NT ? dtvolt[o1 + a] : 0.0;
+      double* x = xs + ln * NR * S + a;
+#pragma unroll
+      for (int v = 0; v < NV; v++) x[v * S] = res[o3 + a + n3 * v] * (v < NM ? dt : dtt);
+      if (!CC) {
+        x[NV * S] = beta[o1 + a];
+        if (NT) x[(NV + 2) * S] = tbeta[o1 + a];
+      }
+    }
   }
   __syncthreads();
-  const int tot = nrow * L;
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    const int r = e / L, a = e - (e / L) * L + 1;
-    const double* dt = r % NV >= 5 ? dtvolt : dtvol;
-    xs[(ll)r * S + a - 1] = res[base3[r] + a] * dt[base1[r] + a];
+  const int ln = threadIdx.x / NV, lv = threadIdx.x - ln * NV;
+  const bool line = ln < nl_here;
+  double* x = xs + (ln * NR + lv) * S;
+  double* g = xs + (ln * NR + NV + (NT && lv >= NM ? 2 : 0)) * S;
+  if (line) {
+    if (CC) strip_forward(x, rt, yt, L, 1, epsc);
+    else strip_forward_v(x, g, g + S, L, 1, lv == 0 || (NT && lv == NM));
   }
+  if (!CC) __syncthreads();
+  if (line) strip_back(x, CC ? rt + 1 : g + S, L, 1, 1);
   __syncthreads();
-  if (threadIdx.x < nrow) il_thomas(xs + (ll)threadIdx.x * S, rt, yt, L, -epsc, 1 + 2 * epsc);
-  __syncthreads();
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    const int r = e / L, a = e - (e / L) * L + 1;
-    res[base3[r] + a] = xs[(ll)r * S + a - 1];
+#pragma unroll 2
+  for (int l2 = threadIdx.x / TA; l2 < nl_here; l2 += 256 / TA) {
+    ll o3, o1;
+    base(l2, o3, o1);
+    for (int a = ta; a < L; a += TA) {
+#pragma unroll
+      for (int v = 0; v < NV; v++) res[o3 + a + n3 * v] = xs[(l2 * NR + v) * S + a];
+    }
   }
 }
 
@@ -1612,21 +1691,29 @@ hipError_t launch_cirs(Solve& s, Level& L, const CirsUpdate* up) {
   double* res = L.f[COSAHIP_RES];
   const double* dt = L.f[COSAHIP_DTVOL];
   const double epsc = 0.25 * (s.par.rat * s.par.rat - 1.0);
-  ll ilines = 0;
-  for (const Blk& b : L.hblk) ilines += (ll)(b.jmax - 1) * (b.kmax - 1) * s.par.nsnap;
+  // i: whole lines resident in LDS where they fit (1400 cells of five
+  // variables with the constant coefficient), else a thread per line and
+  // variable.  Measured (us, the better line kernel of before -> resident):
+  // 192-cell lines of the 193 x 49 x 9 O-grid 83 -> 17, variable coefficients
+  // 84 -> 23 (16 O-grids of 129 x 33 x 5) and 201 -> 58 (SST), the wing's fine
+  // level 203 -> 111, 48 uneven blocks 425 -> 292
   const int mode = s.cirs_i_mode ? s.cirs_i_mode : L.cirs_mode;
-  const bool line = mode == 3 && L.ntile[TK_LINES_IL];
-  const bool iv = line || mode == 2 || (mode == 0 && ilines < CIRS_IV_MAX_LINES);
+  const bool line = mode != 2 && L.ntile[TK_LINES_IL];
   if (line) {
-    const int S = L.il_stride, lpw = L.il_lpw, nv = s.par.npde;
-    const size_t lds = sizeof(double) * (2 * (size_t)S + (size_t)nv * lpw * S) + 2 * sizeof(ll) * nv * lpw;
-    if (nv == 7)
-      hipLaunchKernelGGL(k_cirs_il<7>, grid1(L.ntile[TK_LINES_IL]), dim3(256), lds, s.stream, s.par, L.dblk,
-                         L.tile[TK_LINES_IL], res, dt, L.f[COSAHIP_DTVOLT], L.il_rtab, lpw, S, epsc);
-    else
-      hipLaunchKernelGGL(k_cirs_il<5>, grid1(L.ntile[TK_LINES_IL]), dim3(256), lds, s.stream, s.par, L.dblk,
-                         L.tile[TK_LINES_IL], res, dt, nullptr, L.il_rtab, lpw, S, epsc);
-  } else if (iv && L.ntile[TK_LINES_IV]) {
+    const bool cc = s.par.irsop == 1;
+#define IL(NT, CC)                                                                                                 \
+  hipLaunchKernelGGL((k_cirs_il<5, NT, CC>), grid1(L.ntile[TK_LINES_IL]), dim3(256), L.il_lds, s.stream, s.par,   \
+                     L.dblk, L.tile[TK_LINES_IL], res, dt, L.f[COSAHIP_DTVOLT], L.f[COSAHIP_BETAXI], L.tbeta[0],   \
+                     L.il_rtab, L.il_lpw, L.il_stride, epsc)
+    if (s.par.kom) {
+      if (cc) IL(2, true);
+      else IL(2, false);
+    } else {
+      if (cc) IL(0, true);
+      else IL(0, false);
+    }
+#undef IL
+  } else if (L.ntile[TK_LINES_IV]) {
     if (s.par.npde == 7)
       hipLaunchKernelGGL(k_cirs_iv<7>, grid1(L.ntile[TK_LINES_IV]), dim3(256), 0, s.stream, s.par, L.dblk,
                          L.tile[TK_LINES_IV], res, dt, L.f[COSAHIP_BETAXI], L.f[COSAHIP_DTVOLT], L.tbeta[0], L.cirs_r,
@@ -1636,21 +1723,48 @@ hipError_t launch_cirs(Solve& s, Level& L, const CirsUpdate* up) {
                          L.tile[TK_LINES_IV], res, dt, L.f[COSAHIP_BETAXI], nullptr, nullptr, L.cirs_r, nullptr,
                          epsc);
   }
-  if (!iv && L.ntile[TK_LINES_I])
-    hipLaunchKernelGGL(k_cirs_i<5>, grid1(L.ntile[TK_LINES_I]), dim3(64), 0, s.stream, s.par, L.dblk,
-                       L.tile[TK_LINES_I], res, dt, L.f[COSAHIP_BETAXI], L.cirs_r, 0, epsc);
-  if (s.par.kom && !iv && L.ntile[TK_LINES_I])
-    hipLaunchKernelGGL(k_cirs_i<2>, grid1(L.ntile[TK_LINES_I]), dim3(64), 0, s.stream, s.par, L.dblk,
-                       L.tile[TK_LINES_I], res, L.f[COSAHIP_DTVOLT], L.tbeta[0], L.cirs_r, 5, epsc);
   // j and k sweeps: mean flow and k-omega in one launch per direction
   const double* dtt = L.f[COSAHIP_DTVOLT];
   const CirsUpdate none{};
   // irsop 1 with every line of the level within the LDS tables: the sweep
   // with the forward pass kept in chunks (k_cirs_jkc)
   auto chunked = [&](int dir) {
-    if (s.par.irsop != 1 || s.cirs_jk_chunk == 0 || !L.jk_rtab[dir - 2]) return false;
+    if (s.par.irsop != 1 || s.cirs_jk_mode == 0 || !L.jk_rtab[dir - 2]) return false;
     for (const Blk& b : L.hblk)
       if ((dir == 2 ? b.jmax : b.kmax) - 1 > RTAB_MAX) return false;
+    return true;
+  };
+  // whole lines of a strip in LDS where the level's lines fit (k_cirs_strip)
+  auto strip = [&](int dir, int last, const CirsUpdate* u) {
+    const size_t lds = L.strip_lds[dir - 2];
+    const int nt = L.ntile[dir == 2 ? TK_STRIP_J : TK_STRIP_K];
+    const bool cc = s.par.irsop == 1;
+    if (!lds || !nt || (cc && !L.jk_rtab[dir - 2])) return false;
+    const int nt7 = s.par.kom ? 2 : 0, upd = u ? (u->prim ? 2 : 1) : 0;
+#define STRIP(DIR, NT, UPD, CC)                                                                                  \
+  hipLaunchKernelGGL((k_cirs_strip<DIR, 5, NT, UPD, CC>), dim3(nt), dim3(256), lds, s.stream, s.par, L.dblk,     \
+                     L.tile[DIR == 2 ? TK_STRIP_J : TK_STRIP_K], res, dt, dtt,                                   \
+                     L.f[DIR == 2 ? COSAHIP_BETAETA : COSAHIP_BETAZETA], L.tbeta[DIR - 1], last, epsc,           \
+                     u ? *u : none, L.jk_rtab[DIR - 2])
+#define STRIPC(DIR, NT, UPD)        \
+  do {                              \
+    if (cc) STRIP(DIR, NT, UPD, true); \
+    else STRIP(DIR, NT, UPD, false); \
+  } while (0)
+    if (dir == 2) {
+      if (nt7) STRIPC(2, 2, 0);
+      else STRIPC(2, 0, 0);
+    } else if (nt7) {
+      STRIPC(3, 2, 0);
+    } else if (upd == 2) {
+      STRIPC(3, 0, 2);
+    } else if (upd == 1) {
+      STRIPC(3, 0, 1);
+    } else {
+      STRIPC(3, 0, 0);
+    }
+#undef STRIPC
+#undef STRIP
     return true;
   };
 #define JKC(DIR, NT, UPD, LAST, UP, TK, RT)                                                                       \
@@ -1663,14 +1777,14 @@ hipError_t launch_cirs(Solve& s, Level& L, const CirsUpdate* up) {
                          L.dblk, L.tile[TK], res, dt, NT ? dtt : nullptr, LAST, epsc, UP, RT);                   \
   } while (0)
   if (s.par.kom) {
-    if (L.ntile[TK_LINES_J]) {
+    if (L.ntile[TK_LINES_J] && !strip(2, 0, nullptr)) {
       if (chunked(2)) JKC(2, 2, 0, 0, none, TK_LINES_J, L.jk_rtab[0]);
       else
         hipLaunchKernelGGL((k_cirs_jk<2, 5, 2, 0>), grid1(L.ntile[TK_LINES_J]), dim3(TS), 0, s.stream, s.par, L.dblk,
                            L.tile[TK_LINES_J], res, dt, L.f[COSAHIP_BETAETA], L.cirs_r, dtt, L.tbeta[1], L.cirs_rt, 0,
                            0, epsc, none, L.jk_rtab[0]);
     }
-    if (L.ntile[TK_LINES_K]) {
+    if (L.ntile[TK_LINES_K] && !strip(3, 1, nullptr)) {
       if (chunked(3)) JKC(3, 2, 0, 1, none, TK_LINES_K, L.jk_rtab[1]);
       else
         hipLaunchKernelGGL((k_cirs_jk<3, 5, 2, 0>), grid1(L.ntile[TK_LINES_K]), dim3(TS), 0, s.stream, s.par, L.dblk,
@@ -1678,14 +1792,14 @@ hipError_t launch_cirs(Solve& s, Level& L, const CirsUpdate* up) {
                            1, epsc, none, L.jk_rtab[1]);
     }
   } else {
-    if (L.ntile[TK_LINES_J]) {
+    if (L.ntile[TK_LINES_J] && !strip(2, 0, nullptr)) {
       if (chunked(2)) JKC(2, 0, 0, 0, none, TK_LINES_J, L.jk_rtab[0]);
       else
         hipLaunchKernelGGL((k_cirs_jk<2, 5, 0, 0>), grid1(L.ntile[TK_LINES_J]), dim3(TS), 0, s.stream, s.par, L.dblk,
                            L.tile[TK_LINES_J], res, dt, L.f[COSAHIP_BETAETA], L.cirs_r, nullptr, nullptr, nullptr, 0,
                            0, epsc, none, L.jk_rtab[0]);
     }
-    if (L.ntile[TK_LINES_K]) {
+    if (L.ntile[TK_LINES_K] && !strip(3, 1, up)) {
       const bool ch = chunked(3);
       if (!up) {
         if (ch) JKC(3, 0, 0, 1, none, TK_LINES_K, L.jk_rtab[1]);

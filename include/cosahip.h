@@ -331,15 +331,14 @@ int cosahip_cycle_ready(cosahip_solve* s);
 /* ---- autotuner (no counterpart in the reference) -------------------------
  * Times the interchangeable kernel arrangements on the solve's current
  * state and keeps the fastest: per level the CIRS i-sweep (one thread per
- * line with LDS-staged chunks, or one thread per line and variable), and
+ * line and variable, or whole lines resident in LDS), and
  * for viscous runs the viscous face fluxes (stored then differenced, flux
  * and difference in one line march, or the fluxes of all three directions
  * stored and differenced in one tile pass with the inviscid fluxes).  The
  * arrangements give
  * bit-identical results; the state is not changed (timing runs on a copy of
- * the residual).  choice[0..2]: CIRS i-sweep of levels 1..3 (1 one thread
- * per line with LDS-staged chunks, 2 one thread per line and variable,
- * 3 whole lines resident in LDS -- irsop 1 only --, 0 level absent),
+ * the residual).  choice[0..2]: CIRS i-sweep of levels 1..3 (2 one thread
+ * per line and variable, 3 whole lines resident in LDS, 0 level absent),
  * choice[3]: 1 stored face fluxes, 0 march, 2 tile pass; choice[4..6]: inviscid
  * residual kernel of levels 1..3 (0 generic fused, 1 specialised 31x7
  * tiles with the k-window from LDS/L2, 2 the same with a register
@@ -350,11 +349,12 @@ int cosahip_cycle_ready(cosahip_solve* s);
  * Environment switches at create time take precedence:
  * COSAHIP_RESIDUAL=fused|tile7|tile7reg|tile15|tile7w4|sva7|sva15|sva7w4|tile32w4|sva32|split
  * forces the
- * inviscid residual kernel, COSAHIP_CIRS_I=lds|iv|line forces the i-sweep, COSAHIP_CIRS_IL_LDS sets
+ * inviscid residual kernel, COSAHIP_CIRS_I=iv|line forces the i-sweep, COSAHIP_CIRS_IL_LDS sets
  * the LDS bytes per work-group of the line-resident sweep (4096..65536,
- * default 24576), COSAHIP_VISCOUS=march|fused|faces|tile the viscous
+ * default 40960), COSAHIP_VISCOUS=march|fused|faces|tile the viscous
  * arrangement (default tile, or the autotuner's pick),
- * COSAHIP_CIRS_JK=chunk4|chunk8|plain the irsop 1 j/k sweeps (default chunk4). */
+ * COSAHIP_CIRS_JK=strip|chunk4|chunk8|plain the j/k sweeps (default strip:
+ * whole lines in LDS where they fit; the chunks are for irsop 1).      */
 int cosahip_autotune(cosahip_solve* s, int reps, int32_t* choice);
 
 /* ---- blocks as independent solves (no counterpart in the reference) -----
