@@ -365,6 +365,24 @@ static void add_tiles(std::vector<Tile>& v, int block, ll items, int per) {
   for (ll b0 = 0; b0 < items; b0 += per) v.push_back(Tile{block, (int)b0});
 }
 
+// Work-groups are dealt to the 8 XCDs in turn, each with an L2 of its own:
+// the table is dealt in runs of neighbouring tiles, which share cache lines
+// and halos, to one XCD each.  CIRS strips (64-byte runs of a row, so two
+// strips share most lines): wing fine level j 106 -> 65 us, k 79 -> 52; level 1
+// of 48 uneven blocks j 329 -> 256, k with the update 505 -> 428; the residual
+// tiles 1-7%.  Runs of 16 and 32 were no faster on large levels and slower on
+// small ones; whole eighths of the table left XCDs idle on uneven blocks.  The
+// face and cell kernels and the i-lines did not change.
+static void xcd_order(std::vector<Tile>& v, size_t run) {
+  const size_t nx = 8, n = v.size() / (nx * run) * (nx * run);
+  std::vector<Tile> o(v);
+  for (size_t t = 0; t < n; t++) {
+    const size_t g = t / run, r = t % run;   // run g of XCD g % 8
+    o[((g / nx) * run + r) * nx + g % nx] = v[t];
+  }
+  v.swap(o);
+}
+
 // k_cirs_il (CIRS i-sweep): how many whole lines of all variables (with
 // variable coefficients their coefficients and multipliers too) one
 // work-group keeps in LDS, within s->il_lds bytes (default 40 KB, so that three
@@ -512,6 +530,7 @@ static int build_tables(Solve* s, Level& L, const Level* Lc) {
       add_tiles(L.htile[TK_PROL], b, ns * (ll)((B.imax + 1) / 2) * ((B.jmax + 1) / 2) * ((B.kmax + 1) / 2), TS);
     }
   }
+  for (int k : {(int)TK_STRIP_J, (int)TK_STRIP_K, (int)TK_T32}) xcd_order(L.htile[k], 8);
   for (int k = 0; k < TK_NKIND; k++) {
     if (L.tile[k]) (void)hipFree(L.tile[k]);
     L.tile[k] = nullptr;
