@@ -15,6 +15,78 @@
 namespace cosahip {
 
 // ------------------------------------------------------------------------
+// Quotients and square roots of the face arithmetic.  The fluxes are bound by
+// FP64 instruction issue, and a third of their instructions were divisions
+// and square roots: eleven for each division (two that scale for extreme
+// exponents and one that fixes specials up), about twenty for a root.  Here, in FP64:
+//   * a divisor is inverted once, by Newton-Raphson to the last bits, and
+//     every quotient by it takes three instructions: q = n y, then Markstein's
+//     correction q + (n - q d) y, which rounds to the correctly rounded n / d
+//     (IBM J. Res. Dev. 34 (1990) 111-119); the correction is written as
+//     -(q d - n) y + q, which keeps the sign of an exact zero n (d > 0);
+//   * sqrt(x) comes from the hardware's 1 / sqrt(x) by Goldschmidt's iteration
+//     and two of the same corrections; the refined 1 / sqrt(x) squared is the
+//     start of the inverse of x itself, which saves that its own.
+// The bits are those of the division and the root for operands without
+// extreme exponents (states and their differences: no subnormals, no
+// overflow; below 1e-290 a quotient keeps its absolute, not its relative
+// rounding).  A zero or negative divisor, where the flow state has failed
+// already, gives NaN where the division gives an infinity.
+// FP32 and the contracted build use the operators.
+// Residual of 48 uneven blocks (with the end tests of muscl_face below):
+// VALU instructions 439 M -> 334 M, level 1 1230 -> 1128 us, level 2 160 -> 133;
+// HB O-grid 180 -> 155 us.  It is now bound by the latency of each plane's
+// loads behind its barriers at three waves per SIMD (162 VGPRs): without any
+// Roe flux or limiter division it still took 931 us.  Loading the next plane
+// or the metrics ahead cost the third wave and lost (1180-1450 us).
+#ifdef COSAHIP_CONTRACTED
+constexpr bool FACE_QUOT = false;
+#else
+constexpr bool FACE_QUOT = true;
+#endif
+template <typename T>
+struct Divisor {
+  T d, y;
+  __device__ __forceinline__ explicit Divisor(T d_) : d(d_), y(0) {
+    if constexpr (FACE_QUOT && sizeof(T) == 8) {
+      y = __builtin_amdgcn_rcp(d);
+      y = fma(fma(-d, y, 1.0), y, y);
+      y = fma(fma(-d, y, 1.0), y, y);
+    }
+  }
+  // y0: an approximate inverse of d with at least half its bits right
+  __device__ __forceinline__ Divisor(T d_, T y0) : d(d_), y(y0) {
+    if constexpr (FACE_QUOT && sizeof(T) == 8) y = fma(fma(-d, y, 1.0), y, y);
+  }
+  __device__ __forceinline__ T of(T n) const {
+    if constexpr (FACE_QUOT && sizeof(T) == 8) {
+      const T q = n * y;
+      return fma(-fma(q, d, -n), y, q);
+    } else {
+      return n / d;
+    }
+  }
+};
+// sqrt(x); rs: about 1 / sqrt(x) (FP64)
+template <typename T>
+__device__ __forceinline__ T face_sqrt(T x, T& rs) {
+  if constexpr (FACE_QUOT && sizeof(T) == 8) {
+    const T y = __builtin_amdgcn_rsq(x);
+    T g = x * y, h = y * 0.5;
+    const T r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    g = fma(fma(-g, g, x), h, g);
+    rs = h + h;
+    return g;
+  } else {
+    rs = 0;
+    return sqrt(x);
+  }
+}
+
+// ------------------------------------------------------------------------
 // Roe flux-difference splitting for one face (mean-flow variables).
 template <int NV, typename T = double, int EF = -1>
 __device__ __forceinline__ void roe_face(const Par& p, const T* qr, const T* ql, T kx, T ky, T kz, T ds, T ubn,
@@ -27,7 +99,10 @@ __device__ __forceinline__ void roe_face(const Par& p, const T* qr, const T* ql,
   T unr = ur * kx + vr * ky + wr * kz - ubn;
   T q2r = ur * ur + vr * vr + wr * wr;
   T tker = NV > 5 ? qr[5] : T(0);
-  T h0r = ggm1 * pr / rhor + q2r / 2 + tker;
+  T rsr, rsl;
+  T rhors = face_sqrt(rhor, rsr);
+  const Divisor<T> drr(rhor, rsr * rsr);
+  T h0r = drr.of(ggm1 * pr) + q2r / 2 + tker;
   T rh0r = rhor * h0r;
   T fr0 = rhor * unr;
   T fr1 = (rhor * ur * unr + pr * kx);
@@ -38,7 +113,9 @@ __device__ __forceinline__ void roe_face(const Par& p, const T* qr, const T* ql,
   T unl = ul * kx + vl * ky + wl * kz - ubn;
   T q2l = ul * ul + vl * vl + wl * wl;
   T tkel = NV > 5 ? ql[5] : T(0);
-  T h0l = ggm1 * pl / rhol + q2l / 2 + tkel;
+  T rhols = face_sqrt(rhol, rsl);
+  const Divisor<T> drl(rhol, rsl * rsl);
+  T h0l = drl.of(ggm1 * pl) + q2l / 2 + tkel;
   if (h0lr) {
     h0lr[0] = h0l;
     h0lr[1] = h0r;
@@ -51,20 +128,20 @@ __device__ __forceinline__ void roe_face(const Par& p, const T* qr, const T* ql,
   T fl4 = (rh0l * unl + pl * ubn);
   T drho = rhor - rhol, dp = pr - pl, du = ur - ul, dv = vr - vl, dw = wr - wl, dun = unr - unl;
   T dtke = tker - tkel;
-  T rhols = sqrt(rhol), rhors = sqrt(rhor);
   T rho = rhols * rhors;
-  T denom = rhols + rhors;
-  T u = (rhols * ul + rhors * ur) / denom;
-  T v = (rhols * vl + rhors * vr) / denom;
-  T w = (rhols * wl + rhors * wr) / denom;
+  const Divisor<T> denom(rhols + rhors);
+  T u = denom.of(rhols * ul + rhors * ur);
+  T v = denom.of(rhols * vl + rhors * vr);
+  T w = denom.of(rhols * wl + rhors * wr);
   T un = u * kx + v * ky + w * kz;
-  T h0 = (rhols * h0l + rhors * h0r) / denom;
+  T h0 = denom.of(rhols * h0l + rhors * h0r);
   // mean flow alone: tke = (rhols 0 + rhors 0) / denom is +0 for the
   // positive finite weights, so it is taken as the constant
-  T tke = NV > 5 ? (rhols * tkel + rhors * tker) / denom : T(0);
+  T tke = NV > 5 ? denom.of(rhols * tkel + rhors * tker) : T(0);
   T q2 = u * u + v * v + w * w;
   T a2 = (gamma - 1) * (h0 - q2 / 2 - tke);
-  T a = sqrt(a2);
+  T rsa;
+  T a = face_sqrt(a2, rsa);
   T rm123 = fabs(un - ubn), rm4 = fabs(un + a - ubn), rm5 = fabs(un - a - ubn);
   if (EF != 0 && p.efx_setup_f) {
     T rdelta = (T)p.cntrpy_f * (p.entfx_f_w[0] * (T)p.entfxctf_f + p.entfx_f_w[1] * (sqrt(u * u + v * v + w * w) + a) +
@@ -79,21 +156,23 @@ __device__ __forceinline__ void roe_face(const Par& p, const T* qr, const T* ql,
     if (p.eig_lim_all_f && rm4 <= (T)p.eig_cutoff_f) rm4 = (T)p.eig_cutoff_f;
     if (p.eig_lim_all_f && rm5 <= (T)p.eig_cutoff_f) rm5 = (T)p.eig_cutoff_f;
   }
-  T al1 = rm123 * (drho - dp / a2);
+  const T dpa = Divisor<T>(a2, rsa * rsa).of(dp), rua = Divisor<T>(a, rsa).of(rho * dun);
+  T al1 = rm123 * (drho - dpa);
   T al2 = rm123 * rho;
-  T al3 = rm4 * (dp / a2 + rho * dun / a) / 2;
-  T al4 = rm5 * (dp / a2 - rho * dun / a) / 2;
+  T al3 = rm4 * (dpa + rua) / 2;
+  T al4 = rm5 * (dpa - rua) / 2;
   T df0 = al1 + al3 + al4;
   T df1 = al1 * u + al2 * (du - dun * kx) + al3 * (u + a * kx) + al4 * (u - a * kx);
   T df2 = al1 * v + al2 * (dv - dun * ky) + al3 * (v + a * ky) + al4 * (v - a * ky);
   T df3 = al1 * w + al2 * (dw - dun * kz) + al3 * (w + a * kz) + al4 * (w - a * kz);
   T df4 = al1 * (q2 / 2 + tke) + al2 * (u * du + v * dv + w * dw - un * dun + dtke) + al3 * (h0 + a * un) +
                al4 * (h0 - a * un);
-  F[0] = (fr0 + fl0 - df0) / 2 * ds;
-  F[1] = (fr1 + fl1 - df1) / 2 * ds;
-  F[2] = (fr2 + fl2 - df2) / 2 * ds;
-  F[3] = (fr3 + fl3 - df3) / 2 * ds;
-  F[4] = (fr4 + fl4 - df4) / 2 * ds;
+  const T hds = ds / 2;   // x / 2 * ds and x * (ds / 2) round alike
+  F[0] = (fr0 + fl0 - df0) * hds;
+  F[1] = (fr1 + fl1 - df1) * hds;
+  F[2] = (fr2 + fl2 - df2) * hds;
+  F[3] = (fr3 + fl3 - df3) * hds;
+  F[4] = (fr4 + fl4 - df4) * hds;
 }
 
 // Turbulence part of roflux_b (src/flux.f90:250-383): k and omega upwinded
@@ -112,19 +191,21 @@ __device__ __forceinline__ void roe_turb(const Par& p, const T* qr, const T* ql,
   T tkel = ql[5];
   T fl1 = rhol * unl * tkel, fl2 = rhol * unl * omel;
   T drho = rhor - rhol, dp = pr - pl, dun = unr - unl, dtke = tker - tkel, dome = omer - omel;
-  T rhols = sqrt(rhol), rhors = sqrt(rhor);
+  T rs;
+  T rhols = face_sqrt(rhol, rs), rhors = face_sqrt(rhor, rs);
   T rho = rhols * rhors;
-  T denom = rhols + rhors;
-  T u = (rhols * ul + rhors * ur) / denom;
-  T v = (rhols * vl + rhors * vr) / denom;
-  T w = (rhols * wl + rhors * wr) / denom;
+  const Divisor<T> denom(rhols + rhors);
+  T u = denom.of(rhols * ul + rhors * ur);
+  T v = denom.of(rhols * vl + rhors * vr);
+  T w = denom.of(rhols * wl + rhors * wr);
   T un = u * kx + v * ky + w * kz;
-  T h0 = (rhols * h0l + rhors * h0r) / denom;
-  T tke = (rhols * tkel + rhors * tker) / denom;
-  T ome = (rhols * omel + rhors * omer) / denom;
+  T h0 = denom.of(rhols * h0l + rhors * h0r);
+  T tke = denom.of(rhols * tkel + rhors * tker);
+  T ome = denom.of(rhols * omel + rhors * omer);
   T q2 = u * u + v * v + w * w;
   T a2 = (gamma - 1) * (h0 - q2 / 2 - tke);
-  T a = sqrt(a2);
+  T rsa;
+  T a = face_sqrt(a2, rsa);
   T rm123 = fabs(un - ubn), rm4 = fabs(un + a - ubn), rm5 = fabs(un - a - ubn);
   if (p.efx_setup_t) {
     T rdelta = (T)p.cntrpy_t * (p.entfx_t_w[0] * (T)p.entfxctf_t + p.entfx_t_w[1] * (sqrt(u * u + v * v + w * w) + a) +
@@ -139,27 +220,33 @@ __device__ __forceinline__ void roe_turb(const Par& p, const T* qr, const T* ql,
     if (p.eig_lim_all_t && rm4 <= (T)p.eig_cutoff_t) rm4 = (T)p.eig_cutoff_t;
     if (p.eig_lim_all_t && rm5 <= (T)p.eig_cutoff_t) rm5 = (T)p.eig_cutoff_t;
   }
-  T al1 = rm123 * (drho - dp / a2);
+  const T dpa = Divisor<T>(a2, rsa * rsa).of(dp), rua = Divisor<T>(a, rsa).of(rho * dun);
+  T al1 = rm123 * (drho - dpa);
   T al2 = rm123 * rho;
-  T al3 = rm4 * (dp / a2 + rho * dun / a) / 2;
-  T al4 = rm5 * (dp / a2 - rho * dun / a) / 2;
+  T al3 = rm4 * (dpa + rua) / 2;
+  T al4 = rm5 * (dpa - rua) / 2;
   T df1 = (al1 + al3 + al4) * tke + al2 * dtke;
   T df2 = (al1 + al3 + al4) * ome + al2 * dome;
-  F[5] = (fr1 + fl1 - df1) / 2 * ds;
-  F[6] = (fr2 + fl2 - df2) / 2 * ds;
+  F[5] = (fr1 + fl1 - df1) * (ds / 2);
+  F[6] = (fr2 + fl2 - df2) * (ds / 2);
 }
 
 // ------------------------------------------------------------------------
 // Van Albada slope of the cell between differences d1 (upper face) and d2
 // (lower face), epsq = epslim^2 (limit_i ilim 4, src/flux.f90:3584-3604).
-template <typename T = double>
+// FAST: through Divisor (epsq keeps the divisor away from zero and from the
+// subnormals; launchers take such instances for epslim >= VA_EPS_MIN only).
+constexpr double VA_EPS_MIN = 1e-100;
+template <typename T = double, bool FAST = false>
 __device__ __forceinline__ T va_slope(T epsq, T d1, T d2) {
-  return (d1 * (d2 * d2 + epsq) + d2 * (d1 * d1 + epsq)) / (d1 * d1 + d2 * d2 + 2 * epsq);
+  const T n = d1 * (d2 * d2 + epsq) + d2 * (d1 * d1 + epsq), d = d1 * d1 + d2 * d2 + 2 * epsq;
+  if constexpr (FAST) return Divisor<T>(d).of(n);
+  else return n / d;
 }
 
 // Limited slopes of one variable at face a: dqp(a), dqm(a) from
 // dm1 = dq(a-1), d0 = dq(a), dp1 = dq(a+1)   (limit_i/j/k).
-template <typename T = double>
+template <typename T = double, bool FAST = false>
 __device__ __forceinline__ void limit_face(int ilim, T eps, T rkap, T dm1, T d0, T dp1, T& dqp, T& dqm) {
   if (ilim == 0) {
     T rkp = 1 + rkap, rkm = 1 - rkap;
@@ -194,9 +281,31 @@ __device__ __forceinline__ void limit_face(int ilim, T eps, T rkap, T dm1, T d0,
     dqm = dqmx / 2;
   } else {
     const T epsq = eps * eps;
-    dqp = -va_slope<T>(epsq, dp1, d0) / 2;
-    dqm = va_slope<T>(epsq, d0, dm1) / 2;
+    dqp = -va_slope<T, FAST>(epsq, dp1, d0) / 2;
+    dqm = va_slope<T, FAST>(epsq, d0, dm1) / 2;
   }
+}
+
+// Some lane of the wavefront meets the condition.  The strong-BC cases of the
+// slopes and face states touch only waves at a block's edge; behind this
+// uniform test the others skip their selects and doublings (a tenth of the
+// residual's instructions).
+__device__ __forceinline__ bool any_lane(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
+
+// Strong-BC flags of face a of a line of L faces: fin of face 1, fout of face
+// L, read from the flag planes only there.
+__device__ __forceinline__ void end_flags(const unsigned char* __restrict__ fl, ll in, ll out, int a, int L, bool& fin,
+                                          bool& fout) {
+  fin = fout = false;
+  if (a == 1) fin = fl[in] != 0;
+  if (a == L) fout = fl[out] != 0;
+}
+// The same where the faces next to a matter too (a - 1 .. a + 1).
+__device__ __forceinline__ void near_flags(const unsigned char* __restrict__ fl, ll in, ll out, int a, int L, bool& fin,
+                                           bool& fout) {
+  fin = fout = false;
+  if (a <= 2) fin = fl[in] != 0;
+  if (a >= L - 1) fout = fl[out] != 0;
 }
 
 // Face states qp (right), qm (left) of face a from q(a-2..a+1) of one line.
@@ -206,6 +315,7 @@ __device__ __forceinline__ void limit_face(int ilim, T eps, T rkap, T dm1, T d0,
 template <int NV, typename T = double, int ILIM = -1, int FO = -1>
 __device__ __forceinline__ void muscl_face(const Par& p, int nl, int a, int L, bool fin, bool fout, const T* qm2,
                                            const T* qm1, const T* q0, const T* qp1, T* QR, T* QL) {
+  const bool e1 = a == 1 && fin, eL = a == L && fout;
   if (FO < 0 ? nl >= p.nl_crs : FO == 1) {
 #pragma unroll
     for (int v = 0; v < NV; v++) {
@@ -213,9 +323,24 @@ __device__ __forceinline__ void muscl_face(const Par& p, int nl, int a, int L, b
       QL[v] = qm1[v];
     }
   } else {
-    bool sm1 = (a - 1 == 1 && fin) || (a - 1 == L && fout);
-    bool s0 = (a == 1 && fin) || (a == L && fout);
-    bool sp1 = (a + 1 == 1 && fin) || (a + 1 == L && fout);
+    const bool sm1 = (a - 1 == 1 && fin) || (a - 1 == L && fout);
+    const bool s0 = e1 || eL;
+    const bool sp1 = (a + 1 == 1 && fin) || (a + 1 == L && fout);
+    T dm1[NV], d0[NV], dp1[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      dm1[v] = qm1[v] - qm2[v];
+      d0[v] = q0[v] - qm1[v];
+      dp1[v] = qp1[v] - q0[v];
+    }
+    if (any_lane(sm1 || s0 || sp1)) {
+#pragma unroll
+      for (int v = 0; v < NV; v++) {
+        if (sm1) dm1[v] = dm1[v] * 2;
+        if (s0) d0[v] = d0[v] * 2;
+        if (sp1) dp1[v] = dp1[v] * 2;
+      }
+    }
 #pragma unroll
     for (int v = 0; v < NV; v++) {
       if (v >= 5 && p.foturb) {
@@ -223,26 +348,21 @@ __device__ __forceinline__ void muscl_face(const Par& p, int nl, int a, int L, b
         QL[v] = qm1[v];
         continue;
       }
-      T dm1 = qm1[v] - qm2[v];
-      T d0 = q0[v] - qm1[v];
-      T dp1 = qp1[v] - q0[v];
-      if (sm1) dm1 = (qm1[v] - qm2[v]) * 2;
-      if (s0) d0 = (q0[v] - qm1[v]) * 2;
-      if (sp1) dp1 = (qp1[v] - q0[v]) * 2;
       T dqp, dqm;
-      if (v < 5) limit_face<T>(ILIM < 0 ? p.ilimf : ILIM, (T)p.epslimf, (T)p.rkap, dm1, d0, dp1, dqp, dqm);
-      else limit_face<T>(p.ilimt, (T)p.epslimt, (T)p.rkap, dm1, d0, dp1, dqp, dqm);
+      if (v < 5)
+        limit_face<T, ILIM == 4>(ILIM < 0 ? p.ilimf : ILIM, (T)p.epslimf, (T)p.rkap, dm1[v], d0[v], dp1[v], dqp, dqm);
+      else
+        limit_face<T>(p.ilimt, (T)p.epslimt, (T)p.rkap, dm1[v], d0[v], dp1[v], dqp, dqm);
       QR[v] = q0[v] + dqp;
       QL[v] = qm1[v] + dqm;
     }
   }
-  if (a == 1 && fin) {
+  if (any_lane(e1 || eL)) {
 #pragma unroll
-    for (int v = 0; v < NV; v++) QR[v] = QL[v] = qm1[v];
-  }
-  if (a == L && fout) {
-#pragma unroll
-    for (int v = 0; v < NV; v++) QR[v] = QL[v] = q0[v];
+    for (int v = 0; v < NV; v++) {
+      if (e1) QR[v] = QL[v] = qm1[v];
+      if (eL) QR[v] = QL[v] = q0[v];
+    }
   }
 }
 

@@ -138,8 +138,8 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_tile(Par p, in
     // (b) face fluxes
     if (fr < TJ && fj0 <= jm && fa <= b.imax) {   // i-face a = fa of row fj0
       const int a = fa;
-      const bool fin = fl[fj0 + (ll)(b.jmax + 1) * k] != 0;
-      const bool fout = fl[plI + fj0 + (ll)(b.jmax + 1) * k] != 0;
+      bool fin, fout;
+      near_flags(fl, fj0 + (ll)(b.jmax + 1) * k, plI + fj0 + (ll)(b.jmax + 1) * k, a, b.imax, fin, fout);
       T m2[5], m1[5], z0[5], p1[5], QR[5], QL[5], F[5], kx, ky, kz, ds, ubn;
 #pragma unroll
       for (int v = 0; v < 5; v++) {
@@ -156,8 +156,8 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_tile(Par p, in
     }
     if (tx < TI && ci <= im && cj <= b.jmax) {   // j-face a = cj of column ci
       const int a = cj;
-      const bool fin = fl[offJ + ci + (ll)(b.imax + 1) * k] != 0;
-      const bool fout = fl[offJ + plJ + ci + (ll)(b.imax + 1) * k] != 0;
+      bool fin, fout;
+      near_flags(fl, offJ + ci + (ll)(b.imax + 1) * k, offJ + plJ + ci + (ll)(b.imax + 1) * k, a, b.jmax, fin, fout);
       T m2[5], m1[5], z0[5], p1[5], QR[5], QL[5], F[5], kx, ky, kz, ds, ubn;
 #pragma unroll
       for (int v = 0; v < 5; v++) {
@@ -301,9 +301,9 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_sva(Par p, int
       if (sm1) dm1 = dm1 * 2;
       if (s0) d0 = d0 * 2;
       if (sp1) dp1 = dp1 * 2;
-      hk[v] = va_slope<T>(epsq, dp1, d0) / 2;
+      hk[v] = va_slope<T, true>(epsq, dp1, d0) / 2;
       QR[v] = q0 - hk[v];
-      QL[v] = qm1 + va_slope<T>(epsq, d0, dm1) / 2;
+      QL[v] = qm1 + va_slope<T, true>(epsq, d0, dm1) / 2;
       if (a == 1 && kfin) QR[v] = QL[v] = qm1;
       if (a == b.kmax && kfout) QR[v] = QL[v] = q0;
     }
@@ -327,16 +327,15 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_sva(Par p, int
     //     cells beyond the block compute on unused LDS and are never read
     for (int it = threadIdx.x; it < NI + NJ; it += NT) {
       int c0, st, a, L, ho, hs;
-      bool fin, fout;
+      ll fx, fo;
       if (it < NI) {
         const int r = it / (TI + 2), c = it - r * (TI + 2);
         c0 = (r + 2) * PW + c + 1;
         st = 1;
         a = i0 - 1 + c;
         L = b.imax;
-        const ll fx = min(j0 + r, b.jmax) + (ll)(b.jmax + 1) * k;
-        fin = fl[fx] != 0;
-        fout = fl[plI + fx] != 0;
+        fx = min(j0 + r, b.jmax) + (ll)(b.jmax + 1) * k;
+        fo = plI;
         ho = it;
         hs = NI;
       } else {
@@ -345,23 +344,33 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_sva(Par p, int
         st = PW;
         a = j0 - 1 + r;
         L = b.jmax;
-        const ll fx = offJ + min(i0 + c, b.imax) + (ll)(b.imax + 1) * k;
-        fin = fl[fx] != 0;
-        fout = fl[plJ + fx] != 0;
+        fx = offJ + min(i0 + c, b.imax) + (ll)(b.imax + 1) * k;
+        fo = plJ;
         ho = 5 * NI + jt;
         hs = NJ;
       }
+      bool fin = false, fout = false;
+      if (a <= 1) fin = fl[fx] != 0;
+      if (a >= L - 1) fout = fl[fo + fx] != 0;
       const bool s0 = (a == 1 && fin) || (a == L && fout);            // face a (below the cell)
       const bool s1 = (a + 1 == 1 && fin) || (a + 1 == L && fout);    // face a+1 (above)
+      T d1[5], d2[5];
 #pragma unroll
       for (int v = 0; v < 5; v++) {
         const T* pv = &pl[v][0][0];
         const T qm = pv[c0 - st], qc = pv[c0], qp = pv[c0 + st];
-        T d2 = qc - qm, d1 = qp - qc;
-        if (s0) d2 = d2 * 2;
-        if (s1) d1 = d1 * 2;
-        buf[ho + v * hs] = va_slope<T>(epsq, d1, d2) / 2;
+        d2[v] = qc - qm;
+        d1[v] = qp - qc;
       }
+      if (any_lane(s0 || s1)) {
+#pragma unroll
+        for (int v = 0; v < 5; v++) {
+          if (s0) d2[v] = d2[v] * 2;
+          if (s1) d1[v] = d1[v] * 2;
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < 5; v++) buf[ho + v * hs] = va_slope<T, true>(epsq, d1[v], d2[v]) / 2;
     }
     __syncthreads();
     // (c) face fluxes into registers
@@ -370,32 +379,42 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_sva(Par p, int
     const bool jface = tx < TI && ci <= im && cj <= b.jmax;
     if (iface) {   // i-face a = fa of row fj0
       const int a = fa;
-      const bool fin = fl[fj0 + (ll)(b.jmax + 1) * k] != 0;
-      const bool fout = fl[plI + fj0 + (ll)(b.jmax + 1) * k] != 0;
+      bool fin, fout;
+      end_flags(fl, fj0 + (ll)(b.jmax + 1) * k, plI + fj0 + (ll)(b.jmax + 1) * k, a, b.imax, fin, fout);
       T QR[5], QL[5], kx, ky, kz, ds, ubn;
 #pragma unroll
       for (int v = 0; v < 5; v++) {
         const T qa = pl[v][fr + 2][fc + 2], qm = pl[v][fr + 2][fc + 1];
         QR[v] = qa - hi[v * NI + fr * (TI + 2) + fc + 1];
         QL[v] = qm + hi[v * NI + fr * (TI + 2) + fc];
-        if (a == 1 && fin) QR[v] = QL[v] = qm;
-        if (a == b.imax && fout) QR[v] = QL[v] = qa;
+      }
+      if (any_lane(fin || fout)) {
+#pragma unroll
+        for (int v = 0; v < 5; v++) {
+          if (fin) QR[v] = QL[v] = pl[v][fr + 2][fc + 1];
+          if (fout) QR[v] = QL[v] = pl[v][fr + 2][fc + 2];
+        }
       }
       face_metric<T>(p, si + mo + i2(b, a, fj0, k) * p.lmet, kx, ky, kz, ds, ubn);
       roe_face<5, T, 0>(p, QR, QL, kx, ky, kz, ds, ubn, Fi);
     }
     if (jface) {   // j-face a = cj of column ci
       const int a = cj;
-      const bool fin = fl[offJ + ci + (ll)(b.imax + 1) * k] != 0;
-      const bool fout = fl[offJ + plJ + ci + (ll)(b.imax + 1) * k] != 0;
+      bool fin, fout;
+      end_flags(fl, offJ + ci + (ll)(b.imax + 1) * k, offJ + plJ + ci + (ll)(b.imax + 1) * k, a, b.jmax, fin, fout);
       T QR[5], QL[5], kx, ky, kz, ds, ubn;
 #pragma unroll
       for (int v = 0; v < 5; v++) {
         const T qa = pl[v][ty + 2][tx + 2], qm = pl[v][ty + 1][tx + 2];
         QR[v] = qa - hj[v * NJ + (ty + 1) * TI + tx];
         QL[v] = qm + hj[v * NJ + ty * TI + tx];
-        if (a == 1 && fin) QR[v] = QL[v] = qm;
-        if (a == b.jmax && fout) QR[v] = QL[v] = qa;
+      }
+      if (any_lane(fin || fout)) {
+#pragma unroll
+        for (int v = 0; v < 5; v++) {
+          if (fin) QR[v] = QL[v] = pl[v][ty + 1][tx + 2];
+          if (fout) QR[v] = QL[v] = pl[v][ty + 2][tx + 2];
+        }
       }
       face_metric<T>(p, sj + mo + i2(b, ci, a, k) * p.lmet, kx, ky, kz, ds, ubn);
       roe_face<5, T, 0>(p, QR, QL, kx, ky, kz, ds, ubn, Fj);
@@ -403,22 +422,34 @@ __global__ void __launch_bounds__(32 * (TJ + 1), MINW) k_residual_sva(Par p, int
     if (cell) {   // k-face k+1: h(k) carried, h(k+1) from q(k .. k+2)
       const ll x = i3(b, ci, cj, k);
       const int a = k + 1;
-      const bool s0 = (a == 1 && kfin) || (a == b.kmax && kfout);
-      const bool s1 = (a + 1 == 1 && kfin) || (a + 1 == b.kmax && kfout);
-      T QR[5], QL[5], kx, ky, kz, ds, ubn;
+      const bool s0 = a == b.kmax && kfout, s1 = a + 1 == b.kmax && kfout;   // a >= 2
+      T QR[5], QL[5], q0[5], q1[5], d1[5], d2[5], kx, ky, kz, ds, ubn;
 #pragma unroll
       for (int v = 0; v < 5; v++) {
         const T* qv = qb + n3 * v;
-        const T q0 = pl[v][ty + 2][tx + 2], q1 = qv[x + kstep], q2 = qv[x + 2 * kstep];
-        T d2 = q1 - q0, d1 = q2 - q1;
-        if (s0) d2 = d2 * 2;
-        if (s1) d1 = d1 * 2;
-        const T h1 = va_slope<T>(epsq, d1, d2) / 2;
-        QR[v] = q1 - h1;
-        QL[v] = q0 + hk[v];
+        q0[v] = pl[v][ty + 2][tx + 2];
+        q1[v] = qv[x + kstep];
+        d2[v] = q1[v] - q0[v];
+        d1[v] = qv[x + 2 * kstep] - q1[v];
+      }
+      if (any_lane(s0 || s1)) {
+#pragma unroll
+        for (int v = 0; v < 5; v++) {
+          if (s0) d2[v] = d2[v] * 2;
+          if (s1) d1[v] = d1[v] * 2;
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < 5; v++) {
+        const T h1 = va_slope<T, true>(epsq, d1[v], d2[v]) / 2;
+        QR[v] = q1[v] - h1;
+        QL[v] = q0[v] + hk[v];
         hk[v] = h1;
-        if (a == 1 && kfin) QR[v] = QL[v] = q0;
-        if (a == b.kmax && kfout) QR[v] = QL[v] = q1;
+      }
+      if (any_lane(s0)) {
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+          if (s0) QR[v] = QL[v] = q1[v];
       }
       face_metric<T>(p, sk + mo + i2(b, ci, cj, a) * p.lmet, kx, ky, kz, ds, ubn);
       roe_face<5, T, 0>(p, QR, QL, kx, ky, kz, ds, ubn, Fkn);
@@ -474,7 +505,7 @@ static bool dispatch(Solve& s, Level& L, int variant, const T* q, const T* si, c
   if (!nt) return true;
   const Tile* tl = L.tile[tk];
   const bool fo = L.nl >= p.nl_crs;
-  const bool plain = p.ilimf == 4 && !p.efx_setup_f && !p.eig_limit_f;
+  const bool plain = p.ilimf == 4 && p.epslimf >= VA_EPS_MIN && !p.efx_setup_f && !p.eig_limit_f;
   if (variant == RESID_TILE7) {
     if (!plain) launch_tile<T, 7, -1, -1, -1, 0>(s, L, nt, tl, q, si, sj, sk, res);
     else if (fo) launch_tile<T, 7, 4, 1, 0, 0>(s, L, nt, tl, q, si, sj, sk, res);

@@ -115,8 +115,8 @@ __global__ void __launch_bounds__(32 * (TJ + 1)) k_residual_tile_v(
     //     cell's k-face k + 1
     if (fr < TJ && fj0 <= jm && fa <= b.imax) {
       const int a = fa;
-      const bool fin = fl[fj0 + (ll)(b.jmax + 1) * k] != 0;
-      const bool fout = fl[plI + fj0 + (ll)(b.jmax + 1) * k] != 0;
+      bool fin, fout;
+      near_flags(fl, fj0 + (ll)(b.jmax + 1) * k, plI + fj0 + (ll)(b.jmax + 1) * k, a, b.imax, fin, fout);
       T m2[NV], m1[NV], z0[NV], p1[NV], QR[NV], QL[NV], F[NV], kx, ky, kz, ds, ubn;
 #pragma unroll
       for (int v = 0; v < NV; v++) {
@@ -134,8 +134,8 @@ __global__ void __launch_bounds__(32 * (TJ + 1)) k_residual_tile_v(
     }
     if (tx < TI && ci <= im && cj <= b.jmax) {
       const int a = cj;
-      const bool fin = fl[offJ + ci + (ll)(b.imax + 1) * k] != 0;
-      const bool fout = fl[offJ + plJ + ci + (ll)(b.imax + 1) * k] != 0;
+      bool fin, fout;
+      near_flags(fl, offJ + ci + (ll)(b.imax + 1) * k, offJ + plJ + ci + (ll)(b.imax + 1) * k, a, b.jmax, fin, fout);
       T m2[NV], m1[NV], z0[NV], p1[NV], QR[NV], QL[NV], F[NV], kx, ky, kz, ds, ubn;
 #pragma unroll
       for (int v = 0; v < NV; v++) {
@@ -212,7 +212,7 @@ static void dispatch_v(Solve& s, Level& L, const T* q, const T* si, const T* sj,
   const bool fo = L.nl >= p.nl_crs;
   // van Albada with no entropy fix or eigenvalue floor in either flux:
   // specialised; everything else through the run-time flags
-  const bool plain = p.ilimf == 4 && !p.efx_setup_f && !p.eig_limit_f;
+  const bool plain = p.ilimf == 4 && p.epslimf >= VA_EPS_MIN && !p.efx_setup_f && !p.eig_limit_f;
   if (!plain) launch_v<T, NV, VIS, -1, -1, -1>(s, L, q, si, sj, sk, res, vf, vslot);
   else if (fo) launch_v<T, NV, VIS, 4, 1, 0>(s, L, q, si, sj, sk, res, vf, vslot);
   else launch_v<T, NV, VIS, 4, 0, 0>(s, L, q, si, sj, sk, res, vf, vslot);

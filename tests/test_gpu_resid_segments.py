@@ -43,6 +43,18 @@ def test_segments_same_bits(dims, monkeypatch):
     assert np.array_equal(_residual(c, q0, monkeypatch).view(np.uint64), ref.view(np.uint64))
 
 
+@pytest.mark.parametrize("eps", [1e-6, 1e-99, 1e-160])
+def test_limiter_floor_same_bits(eps, monkeypatch):
+    """Uniform lines (zero differences) and limiter constants on both sides of
+    the one below which the quotient by the reciprocal would meet subnormals."""
+    c = cases.channel_case([(34, 12, 9)], nlevel=1, irsop=1, cfl=2.0, cfl_irs=4.0, epslimf=eps)
+    q0 = c.freestream()
+    ref = _residual(c, q0, monkeypatch, COSAHIP_RESIDUAL="split")
+    got = _residual(c, q0, monkeypatch)
+    assert np.isfinite(ref).all()
+    assert np.array_equal(got, ref)
+
+
 @pytest.mark.parametrize("mode", ["faces", "march"])
 def test_viscous_default_same_bits(mode, monkeypatch):
     c = cases.two_block_case(ni=34, nj=16, nk=13, nlevel=1, distort=0.1, wall=1500, irsop=1, cfl_irs=2.5, cfl=1.5,
