@@ -196,6 +196,12 @@ static Par make_par(const cosahip_config& c) {
   p.gkw = c.gkw;
   p.prdlim = c.prdlim;
   p.roughk = c.roughk;
+  p.inv_gm1 = 1 / (c.gamma - 1);
+  if (c.viscous) {   // positive (check_config)
+    p.inv_reyno = 1 / c.reyno;
+    p.inv_pranl = 1 / c.pranl;
+    p.inv_prant = 1 / c.prant;
+  }
   p.qmin6 = c.qmin[5];
   p.qmin7 = c.qmin[6];
   return p;

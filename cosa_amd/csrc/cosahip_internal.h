@@ -34,6 +34,7 @@ struct Par {
   int ilimf, irsop, nl_crs;
   double gamma, rkap, epslimf;
   double gam_gm1;   // gamma / (gamma - 1), the same correctly rounded quotient the flux evaluates
+  double inv_gm1, inv_reyno, inv_pranl, inv_prant;   // 1 / (gamma - 1) and so on, for Divisor::constant
   double cfl, rat, psirs;
   int efx_setup_f, efx_all_f, eig_limit_f, eig_lim_all_f;
   int entfx_f_w[3];

@@ -3,6 +3,7 @@
 // COSA's pseudo-time loop, for gfx950.  Each kernel restates one reference
 // routine (cited); arithmetic keeps the reference's operation order.
 #include "kernels.h"
+#include "quot.h"
 
 namespace cosahip {
 
@@ -905,7 +906,7 @@ __global__ void __launch_bounds__(256) k_bc(Par p, const Blk* __restrict__ blks,
     }
     if (p.kom) {
       const double tw = pw * p.gamma / rhow;
-      const double muw = (p.stemp + 1) / (tw + p.stemp) * pow(tw, 1.5);
+      const double muw = (p.stemp + 1) / (tw + p.stemp) * pow32(tw);
       const double dn = dist[b.o1 + i1(b, in, jn, kn)];
       double omew;
       if (p.wallwilc) {

@@ -487,27 +487,26 @@ __global__ void __launch_bounds__(256) k_lambda_deltat(Par p, const Blk* __restr
     // k-omega; the +1 neighbour's temperature divides by the -1 neighbour's
     // density, as in the reference
     const double gamma = p.gamma;
-    const double t0 = gamma * pp / rho;
-    const double mu = (p.stemp + 1.0) / (t0 + p.stemp) * pow(t0, 1.5);
+    const Divisor<double> dl = Divisor<double>::constant(p.pranl, p.inv_pranl),
+                          dt = Divisor<double>::constant(p.prant, p.inv_prant),
+                          dr = Divisor<double>::constant(p.reyno, p.inv_reyno);
+    const double mu = suth<double>(p, gamma * pp / rho);
     const double* mb = p.kom ? mut + b.o3 * p.nsnap + n3 * (ll)n : nullptr;
     const double mutc = p.kom ? mb[c] : 0.0;
     const double vc = vol[b.o1 + i1(b, i, j, k)];
+    const Divisor<double> drv(rho * vc);
     const ll st[3] = {1, (ll)(b.imax + 3), (ll)(b.imax + 3) * (b.jmax + 3)};
     const double ar_[3] = {axi, aeta, azeta};
 #pragma unroll
     for (int d = 0; d < 3; d++) {
       const ll cm = c - st[d], cp = c + st[d];
-      const double rhom = qb[cm], pm = qb[cm + 4 * n3];
-      const double tm = gamma * pm / rhom;
-      const double mum = (p.stemp + 1.0) / (tm + p.stemp) * pow(tm, 1.5);
-      const double mutm = p.kom ? mb[cm] : 0.0;
-      const double ppn = qb[cp + 4 * n3];
-      const double tp = gamma * ppn / rhom;
-      const double mup = (p.stemp + 1.0) / (tp + p.stemp) * pow(tp, 1.5);
-      const double mutp = p.kom ? mb[cp] : 0.0;
+      const double rhom = qb[cm], pm = qb[cm + 4 * n3], ppn = qb[cp + 4 * n3];
+      const Divisor<double> drm(rhom);
+      const double mum = suth<double>(p, drm.of(gamma * pm)), mup = suth<double>(p, drm.of(gamma * ppn));
+      const double mutm = p.kom ? mb[cm] : 0.0, mutp = p.kom ? mb[cp] : 0.0;
       const double mud = (mum + 2 * mu + mup) / 4;
       const double mutd = (mutm + 2 * mutc + mutp) / 4;
-      lv[d] = p.cdff * ar_[d] * ar_[d] * gamma * p.machfs / p.reyno * (mud / p.pranl + mutd / p.prant) / (rho * vc);
+      lv[d] = drv.of(dr.of(p.cdff * ar_[d] * ar_[d] * gamma * p.machfs) * (dl.of(mud) + dt.of(mutd)));
     }
     // irsop 5/6 take the viscous radii into the smoothing, not the time
     // step (src/cosa.f90:4831-4890)

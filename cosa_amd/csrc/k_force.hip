@@ -10,6 +10,7 @@
 //   k_force_coef   one thread per (snapshot, surface): the coefficients of
 //                  each block, then their sum over the blocks in order.
 #include "kernels.h"
+#include "quot.h"
 #include "viscous.h"
 
 namespace cosahip {
@@ -79,7 +80,7 @@ __global__ void __launch_bounds__(256) k_force_terms(Par p, const Blk* __restric
   const double etax = e3[0], etay = e3[1], etaz = e3[2];
   const double rhow = r1;
   const double tw = pw * gamma / rhow;
-  const double muw = (p.stemp + 1) / (tw + p.stemp) * pow(tw, 1.5);
+  const double muw = (p.stemp + 1) / (tw + p.stemp) * pow32(tw);
   int c1[3] = {c[0], c[1], c[2]}, c2[3] = {c[0], c[1], c[2]};
   c1[idir - 1] += sgn;
   c2[idir - 1] += 2 * sgn;

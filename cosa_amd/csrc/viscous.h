@@ -3,12 +3,13 @@
 // kernels (k_flux.hip).
 #pragma once
 #include "cosahip_internal.h"
+#include "quot.h"
 
 namespace cosahip {
 
 template <typename T>
 __device__ __forceinline__ T suth(const Par& p, T t) {
-  return ((T)p.stemp + 1) / (t + (T)p.stemp) * pow(t, T(1.5));
+  return Divisor<T>(t + (T)p.stemp).of((T)p.stemp + 1) * pow32(t);
 }
 
 // strong-BC flag byte of the face of direction DIR at position a (1 or L)
@@ -139,7 +140,9 @@ __device__ __forceinline__ void viscous_face(const Par& p, const Blk& b, int i, 
   const T kx = s[0], ky = s[1], kz = s[2], ds = s[3];
   const T gamma = (T)p.gamma;
   const T rho = qf[0], u = qf[1], v = qf[2], w = qf[3], pr = qf[4];
-  const T tmp = gamma * pr / rho;
+  const Divisor<T> drho(rho), dpr(pr), d3 = Divisor<T>::constant(3, 1.0 / 3.0),
+                   drey = Divisor<T>::constant((T)p.reyno, p.inv_reyno);
+  const T tmp = drho.of(gamma * pr);
   const T mu = suth<T>(p, tmp);
   const T uxi = dd[0][1], ueta = dd[1][1], uzeta = dd[2][1];
   const T vxi = dd[0][2], veta = dd[1][2], vzeta = dd[2][2];
@@ -161,12 +164,13 @@ __device__ __forceinline__ void viscous_face(const Par& p, const Blk& b, int i, 
     const T tke = qf[5];
     const T fact = T(2.0 / 3.0);
     const T divt = (dudx + dvdy + dwdz) * (T)p.turcmp;
-    const T ttxx = 2 * mutf * (dudx - divt / 3);
+    const T divt3 = d3.of(divt);
+    const T ttxx = 2 * mutf * (dudx - divt3);
     const T ttxy = mutf * (dudy + dvdx);
     const T ttxz = mutf * (dudz + dwdx);
-    const T ttyy = 2 * mutf * (dvdy - divt / 3);
+    const T ttyy = 2 * mutf * (dvdy - divt3);
     const T ttyz = mutf * (dvdz + dwdy);
-    const T ttzz = 2 * mutf * (dwdz - divt / 3);
+    const T ttzz = 2 * mutf * (dwdz - divt3);
     const T r1 = mr * ttxx - fact * rho * tke;
     const T r2 = mr * ttxy;
     const T r3 = mr * ttxz;
@@ -207,28 +211,30 @@ __device__ __forceinline__ void viscous_face(const Par& p, const Blk& b, int i, 
       sk = f1 * (T)p.sigk1 + (1 - f1) * (T)p.sigk2;
       sw = f1 * (T)p.sigw1 + (1 - f1) * (T)p.sigw2;
     }
-    const T ctke = (mu + sk * mutf) * (T)p.machfs / (T)p.reyno;
-    const T come = (mu + sw * mutf) * (T)p.machfs / (T)p.reyno;
+    const T ctke = drey.of((mu + sk * mutf) * (T)p.machfs);
+    const T come = drey.of((mu + sw * mutf) * (T)p.machfs);
     F[4] = -(ctke * (dtkedx * kx + dtkedy * ky + dtkedz * kz) * ds);
     F[5] = -(ctke * (dtkedx * kx + dtkedy * ky + dtkedz * kz) * ds);
     // as in the reference: dk/dz in place of domega/dz
     F[6] = -(come * (domedx * kx + domedy * ky + dtkedz * kz) * ds);
   }
   // laminar stresses and heat flux (common part of vflux_b)
-  const T txi = tmp * (dd[0][4] / pr - dd[0][0] / rho);
-  const T teta = tmp * (dd[1][4] / pr - dd[1][0] / rho);
-  const T tzeta = tmp * (dd[2][4] / pr - dd[2][0] / rho);
+  const T txi = tmp * (dpr.of(dd[0][4]) - drho.of(dd[0][0]));
+  const T teta = tmp * (dpr.of(dd[1][4]) - drho.of(dd[1][0]));
+  const T tzeta = tmp * (dpr.of(dd[2][4]) - drho.of(dd[2][0]));
   const T dtdx = txi * xix + teta * etax + tzeta * zetax;
   const T dtdy = txi * xiy + teta * etay + tzeta * zetay;
   const T dtdz = txi * xiz + teta * etaz + tzeta * zetaz;
-  const T divv = dudx + dvdy + dwdz;
-  const T txx = mr * 2 * mu * (dudx - divv / 3);
+  const T divv = dudx + dvdy + dwdz, divv3 = d3.of(divv);
+  const T txx = mr * 2 * mu * (dudx - divv3);
   const T txy = mr * mu * (dudy + dvdx);
   const T txz = mr * mu * (dudz + dwdx);
-  const T tyy = mr * 2 * mu * (dvdy - divv / 3);
+  const T tyy = mr * 2 * mu * (dvdy - divv3);
   const T tyz = mr * mu * (dvdz + dwdy);
-  const T tzz = mr * 2 * mu * (dwdz - divv / 3);
-  const T cq = mr * (mu / (T)p.pranl + mutf / (T)p.prant) / (gamma - 1);
+  const T tzz = mr * 2 * mu * (dwdz - divv3);
+  const T cq = Divisor<T>::constant(gamma - 1, p.inv_gm1)
+                   .of(mr * (Divisor<T>::constant((T)p.pranl, p.inv_pranl).of(mu) +
+                             Divisor<T>::constant((T)p.prant, p.inv_prant).of(mutf)));
   const T qx = -(cq * dtdx), qy = -(cq * dtdy), qz = -(cq * dtdz);
   F[0] = 0;
   F[1] = F[1] - (txx * kx + txy * ky + txz * kz) * ds;
