@@ -89,7 +89,7 @@ static void free_level(Level& L) {
   void* ptrs[] = {L.dblk, L.dq, L.work1, L.cirs_r, L.cirs_rt, L.rms_part, L.sbc, L.sbc_doff, L.dpatch, L.dcut,
                   L.vflux, L.tbeta[0], L.tbeta[1], L.tbeta[2], L.h0tab, L.dxd, L.q32, L.m32[0], L.m32[1], L.m32[2],
                   L.dxd32, L.mut32, L.dwall, L.fterms, L.fsums, L.fcoef, L.fgeom, L.dqc, L.il_rtab, L.cmet,
-                  L.cmet32, L.ptile, L.jk_rtab[0], L.jk_rtab[1]};
+                  L.cmet32, L.ptile, L.ctile, L.jk_rtab[0], L.jk_rtab[1]};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (float* p : L.xd32)
@@ -594,6 +594,52 @@ static bool cut_in_bounds(const Blk& b1, const Blk& b2, const int32_t* t, int n2
 
 static ll field_size(const Solve* s, const Level& L, int field);
 
+// Every face-halo cell of every block is set by exactly one point of one patch
+// or cut, and no block is one cell thick: then the halo fill and bprtest may
+// run as one launch (k_halo) -- no order between patches and cuts matters, and
+// the cells they set are all the halo cells bprtest looks at.
+static bool halos_set_once(const Level& L) {
+  if (L.thin) return false;
+  std::vector<std::vector<unsigned char>> hit(6 * (size_t)L.nblocks);
+  auto mark = [&](int block, int idir, int inout, int c2lo, int c2hi, int c3lo, int c3hi) {
+    // transverse extents in the cyclic order of the record
+    const Blk& B = L.hblk[block];
+    const int ext[4] = {0, B.imax - 1, B.jmax - 1, B.kmax - 1};
+    const int e2 = ext[idir % 3 + 1], e3 = ext[(idir + 1) % 3 + 1];
+    auto& h = hit[6 * (size_t)block + 2 * (idir - 1) + (inout == 1 ? 0 : 1)];
+    if (h.empty()) h.assign((size_t)e2 * e3, 0);
+    if (c2lo < 1 || c3lo < 1 || c2hi > e2 || c3hi > e3) return false;
+    for (int c3 = c3lo; c3 <= c3hi; c3++)
+      for (int c2 = c2lo; c2 <= c2hi; c2++)
+        if (h[(size_t)(c3 - 1) * e2 + c2 - 1]++) return false;
+    return true;
+  };
+  for (const PatchRec& r : L.hpatch) {
+    const int i2 = r.t[1] % 3 + 1, i3 = (r.t[1] + 1) % 3 + 1;
+    if (!mark(r.block, r.t[1], r.t[2], r.t[2 * i2 + 1], r.t[2 * i2 + 2], r.t[2 * i3 + 1], r.t[2 * i3 + 2])) return false;
+  }
+  for (const CutRec& r : L.hcut) {
+    const int i2 = r.t[1] % 3 + 1, i3 = (r.t[1] + 1) % 3 + 1;
+    const int a2 = r.t[2 * i2 + 1], b2 = r.t[2 * i2 + 2], a3 = r.t[2 * i3 + 1], b3 = r.t[2 * i3 + 2];
+    if (!mark(r.b1, r.t[1], r.t[2], std::min(a2, b2), std::max(a2, b2), std::min(a3, b3), std::max(a3, b3))) return false;
+    // the sources: interior cells of block 2 (cut_in_bounds allows its halos)
+    const Blk& B2 = L.hblk[r.b2];
+    const int ext[4] = {0, B2.imax - 1, B2.jmax - 1, B2.kmax - 1};
+    for (int m = 1; m <= 2; m++) {
+      const int d = r.t[17 + (r.t[1] + m - 1) % 3 + 1], len = m == 1 ? b2 - a2 : b3 - a3;
+      const int lo = r.t[10 + 2 * d], sg = r.t[11 + 2 * d] > lo ? 1 : -1;
+      const int hi = lo + sg * std::abs(len);
+      if (std::min(lo, hi) < 1 || std::max(lo, hi) > ext[d]) return false;
+    }
+  }
+  for (const auto& h : hit) {
+    if (h.empty()) return false;
+    for (unsigned char c : h)
+      if (c != 1) return false;
+  }
+  return true;
+}
+
 // FP32 shadows of the level's primitive q and face metrics (FP32-residual mode)
 static int alloc_fp32(Solve* s, Level& L) {
   if (L.q32) return COSAHIP_OK;
@@ -785,7 +831,6 @@ extern "C" int cosahip_define_level(cosahip_solve* h, int nl, int nblocks, const
     if (!cut_in_bounds(L.hblk[r.b1], L.hblk[r.b2], t, r.n2, r.count))
       return fail(s, COSAHIP_ERR_ARG, "cutopo: cut maps outside a block");
     L.hcut.push_back(r);
-    L.maxcut = std::max(L.maxcut, r.count);
   }
   CK(upload_vec(&L.dblk, L.hblk));
   CK(upload_vec(&L.dpatch, L.hpatch));
@@ -799,6 +844,14 @@ extern "C" int cosahip_define_level(cosahip_solve* h, int nl, int nblocks, const
   }
   CK(upload_vec(&L.ptile, L.hptile));
   CK(upload_vec(&L.dcut, L.hcut));
+  L.hctile.clear();
+  L.ctile_first.assign(1, 0);
+  for (size_t ic = 0; ic < L.hcut.size(); ic++) {
+    add_tiles(L.hctile, (int)ic, (ll)L.hcut[ic].count * s->par.nsnap, TS);
+    L.ctile_first.push_back((int)L.hctile.size());
+  }
+  CK(upload_vec(&L.ctile, L.hctile));
+  L.halo_once = halos_set_once(L);
   CK(upload_vec(&L.sbc, sbc));
   CK(upload_vec(&L.sbc_doff, L.sbc_off));
   // fields
@@ -1983,8 +2036,7 @@ static int smooth_core(Solve* s, int nl, int from_fine, int to_coarse, int niter
       q_prim = false;
       {
         TimeScope t(*s, COSAHIP_FAM_HALO, cs);
-        CK(launch_bc(*s, L, q));
-        CK(launch_cut(*s, L, q));
+        CK(launch_halo(*s, L, q, true, seq));
         CK(launch_halo_f32(*s, L));
       }
       if (komega(c) && mgit == 1 && iter == 1 && irk == 1 && from_fine && !c.prd_all_lvls) {
@@ -1993,7 +2045,7 @@ static int smooth_core(Solve* s, int nl, int from_fine, int to_coarse, int niter
         if (c.kom_sst) CK(launch_sst_first_mut(*s, L));
         else CK(launch_tur_vis(*s, L, q));
       }
-      {
+      if (!L.halo_once) {
         TimeScope t(*s, COSAHIP_FAM_OTHER, cs);
         CK(launch_prtest(*s, L, q, seq));
       }
@@ -2153,8 +2205,7 @@ static int prolong_core(Solve* s, int nl) {
   double* arrs[2] = {L2.f[COSAHIP_QOLD], L2.f[COSAHIP_Q]};
   for (double* a : arrs) {
     CK(launch_cons2prim(*s, L2, a));
-    CK(launch_bc(*s, L2, a));
-    CK(launch_cut(*s, L2, a));
+    CK(launch_halo(*s, L2, a));
     CK(launch_prim2cons(*s, L2, a));
     CK(launch_edges_corners(*s, L2, a));
   }

@@ -784,6 +784,12 @@ __global__ void __launch_bounds__(256) k_rms_final(const double* __restrict__ pa
 }
 
 // ---- bprtest (src/cosa.f90:960-1120): first offender in loop order ----
+__device__ __forceinline__ unsigned long long prtest_key(const Par& p, int block, int n, int reg, int loc,
+                                                         unsigned long long kind, int stage_seq) {
+  const unsigned long long seq = stage_seq < 511 ? (unsigned long long)stage_seq : 511ull;
+  const unsigned long long pos = ((unsigned long long)block * p.nsnap + n) * 5 + reg;
+  return (seq << 55) | (pos << 29) | ((unsigned long long)(loc & 0x7FFFFFF) << 2) | kind;
+}
 __global__ void __launch_bounds__(256) k_prtest(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                 const double* __restrict__ q, int stage_seq,
                                                 unsigned long long* __restrict__ flag) {
@@ -798,10 +804,7 @@ __global__ void __launch_bounds__(256) k_prtest(Par p, const Blk* __restrict__ b
   if (pp <= p.qmin5) kind = 1;
   else if (rho <= p.qmin1) kind = 2;
   if (!kind) return;
-  const unsigned long long seq = stage_seq < 511 ? (unsigned long long)stage_seq : 511ull;
-  const unsigned long long pos = ((unsigned long long)t.block * p.nsnap + n) * 5 + reg;
-  const unsigned long long key = (seq << 55) | (pos << 29) | ((unsigned long long)(loc & 0x7FFFFFF) << 2) | kind;
-  atomicMin(flag, key);
+  atomicMin(flag, prtest_key(p, t.block, n, reg, loc, kind, stage_seq));
 }
 
 // ---- boundary conditions (src/bc.f90) ----
@@ -812,18 +815,16 @@ __device__ __forceinline__ void bc_ijk(int ic1, int ic2, int ic3, int a, int i2_
 }
 __device__ __forceinline__ int cycd(int d, int m) { return (d - 1 + m - 1) % 3 + 1; }
 
-__global__ void __launch_bounds__(256) k_bc(Par p, const Blk* __restrict__ blks, const PatchRec* __restrict__ pr,
-                                            const Tile* __restrict__ tiles, double* __restrict__ q,
-                                            const double* __restrict__ si, const double* __restrict__ sj,
-                                            const double* __restrict__ sk, const double* __restrict__ dist,
-                                            const double* __restrict__ qfb) {
-  const Tile tl = tiles[blockIdx.x];
-  const PatchRec rec = pr[tl.block];
-  const int item = tl.base + threadIdx.x;
-  if (item >= rec.count * p.nsnap) return;
-  const Blk b = blks[rec.block];
-  const int n = item / rec.count;
-  const int loc = item - n * rec.count;
+// One face point of a patch: both halo layers set from the interior.  h: the
+// two halo cells.
+struct HaloCells {
+  int n, i[2], j[2], k[2];
+};
+__device__ __forceinline__ void bc_point(const Par& p, const PatchRec& rec, const Blk& b, int n, int loc,
+                                         double* __restrict__ q, const double* __restrict__ si,
+                                         const double* __restrict__ sj, const double* __restrict__ sk,
+                                         const double* __restrict__ dist, const double* __restrict__ qfb,
+                                         HaloCells& h) {
   const int idir = rec.t[1], inrout = rec.t[2];
   const int ic1 = cycd(idir, 1), ic2 = cycd(idir, 2), ic3 = cycd(idir, 3);
   // every face point is set from the interior alone, so the order of the
@@ -852,6 +853,7 @@ __global__ void __launch_bounds__(256) k_bc(Par p, const Blk* __restrict__ blks,
   bc_ijk(ic1, ic2, ic3, ibcpt, i2_, i3_, ib, jb, kb);
   bc_ijk(ic1, ic2, ic3, ibcpt2, i2_, i3_, ib2, jb2, kb2);
   bc_ijk(ic1, ic2, ic3, ibcn, i2_, i3_, in, jn, kn);
+  h = HaloCells{n, {ib, ib2}, {jb, jb2}, {kb, kb2}};
   double* qb = qblk(p, b, q, n);
   const ll n3 = n3of(b);
   const ll xb = i3(b, ib, jb, kb), xb2 = i3(b, ib2, jb2, kb2), xn = i3(b, in, jn, kn);
@@ -936,7 +938,6 @@ __global__ void __launch_bounds__(256) k_bc(Par p, const Blk* __restrict__ blks,
     // freestream of the patch's block (blocks may be independent solves)
     const double* qfst = qfb + 5 * rec.block;
     const double gamma = p.gamma;
-    const double sinf = p.pinf / pow(p.rhoinf, gamma);
     double sx = sm[0] * sgnm, sy = sm[1] * sgnm, sz = sm[2] * sgnm;
     double qext = qb[xn + n3] * sx + qb[xn + 2 * n3] * sy + qb[xn + 3 * n3] * sz;
     double qinf = qfst[1] * sx + qfst[2] * sy + qfst[3] * sz;
@@ -948,12 +949,12 @@ __global__ void __launch_bounds__(256) k_bc(Par p, const Blk* __restrict__ blks,
     double qdotn = (rext + rinf) / 2;
     double a = (gamma - 1) * (rext - rinf) / 4;
     double mach = qdotn / a;
-    double sext = pext / pow(rhoext, gamma);
     if (qdotn <= 0.0) {
       if (fabs(mach) >= 1.0) {
         for (int v = 0; v < 5; v++) hv[v] = qfst[v];
         set = true;
       } else if (fabs(mach) < 1.0) {
+        const double sinf = p.pinf / pow(p.rhoinf, gamma);
         double rhobc = pow(a * a / (gamma * sinf), 1.0 / (gamma - 1));
         double pb = rhobc * a * a / gamma;
         hv[0] = rhobc;
@@ -968,6 +969,7 @@ __global__ void __launch_bounds__(256) k_bc(Par p, const Blk* __restrict__ blks,
         for (int v = 0; v < 5; v++) hv[v] = qb[xn + v * n3];
         set = true;
       } else if (fabs(mach) < 1.0) {
+        const double sext = pext / pow(rhoext, gamma);
         double rhobc = pow(a * a / (gamma * sext), 1.0 / (gamma - 1));
         double pb = rhobc * a * a / gamma;
         hv[0] = rhobc;
@@ -1023,13 +1025,25 @@ __global__ void __launch_bounds__(256) k_bc(Par p, const Blk* __restrict__ blks,
     }
 }
 
+__global__ void __launch_bounds__(256) k_bc(Par p, const Blk* __restrict__ blks, const PatchRec* __restrict__ pr,
+                                            const Tile* __restrict__ tiles, double* __restrict__ q,
+                                            const double* __restrict__ si, const double* __restrict__ sj,
+                                            const double* __restrict__ sk, const double* __restrict__ dist,
+                                            const double* __restrict__ qfb) {
+  const Tile tl = tiles[blockIdx.x];
+  const PatchRec rec = pr[tl.block];
+  const int item = tl.base + threadIdx.x;
+  if (item >= rec.count * p.nsnap) return;
+  const Blk b = blks[rec.block];
+  const int n = item / rec.count;
+  HaloCells h;
+  bc_point(p, rec, b, n, item - n * rec.count, q, si, sj, sk, dist, qfb, h);
+}
+
 // ---- cut_q, same-device copy (src/bc.f90:1894-2141) ----
-__global__ void __launch_bounds__(256) k_cut(Par p, const Blk* __restrict__ blks, const CutRec* __restrict__ cr,
-                                             int first, double* __restrict__ q) {
-  const CutRec rec = cr[first + blockIdx.y];
-  const int item = blockIdx.x * blockDim.x + threadIdx.x;
-  if (item >= rec.count) return;
-  const Blk b1 = blks[rec.b1], b2 = blks[rec.b2];
+// One point and snapshot of a cut record: both halo layers of block 1.
+__device__ __forceinline__ void cut_point(const Par& p, const CutRec& rec, const Blk& b1, const Blk& b2, int n,
+                                          int item, double* __restrict__ q, HaloCells& h) {
   const int* t = rec.t;
   const int idir1 = t[1], inout1 = t[2], idir2 = t[10], inout2 = t[11];
   int istr1[4], iend1[4], istr2[4], iend2[4], iord[4];
@@ -1056,14 +1070,100 @@ __global__ void __launch_bounds__(256) k_cut(Par p, const Blk* __restrict__ blks
   const ll n31 = n3of(b1), n32 = n3of(b2);
   const ll d1 = i3(b1, ii1, jj1, kk1), d2 = i3(b1, ii2, jj2, kk2);
   const ll s1 = i3(b2, in1, jn1, kn1), s2 = i3(b2, in2, jn2, kn2);
-  for (int n = 0; n < p.nsnap; n++) {
-    double* q1 = qblk(p, b1, q, n);
-    const double* q2 = qblk(p, b2, q, n);
-    for (int v = 0; v < p.npde; v++) {
-      q1[d1 + v * n31] = q2[s1 + v * n32];
-      q1[d2 + v * n31] = q2[s2 + v * n32];
-    }
+  h = HaloCells{n, {ii1, ii2}, {jj1, jj2}, {kk1, kk2}};
+  double* q1 = qblk(p, b1, q, n);
+  const double* q2 = qblk(p, b2, q, n);
+  for (int v = 0; v < p.npde; v++) {
+    q1[d1 + v * n31] = q2[s1 + v * n32];
+    q1[d2 + v * n31] = q2[s2 + v * n32];
   }
+}
+// tiles: (cut record, first item), items count x snapshots
+__global__ void __launch_bounds__(256) k_cut(Par p, const Blk* __restrict__ blks, const CutRec* __restrict__ cr,
+                                             const Tile* __restrict__ tiles, double* __restrict__ q) {
+  const Tile tl = tiles[blockIdx.x];
+  const CutRec rec = cr[tl.block];
+  const int item = tl.base + threadIdx.x;
+  if (item >= rec.count * p.nsnap) return;
+  const int n = item / rec.count;
+  HaloCells h;
+  cut_point(p, rec, blks[rec.b1], blks[rec.b2], n, item - n * rec.count, q, h);
+}
+
+// bprtest's test of one cell of block `block` (see k_prtest), the cell by its
+// indices: the inverse of halo_of
+__device__ __forceinline__ void prtest_cell(const Par& p, const Blk& b, int block, int n, int i, int j, int k,
+                                            const double* q, int stage_seq, unsigned long long* __restrict__ flag) {
+  const double* qb = qblk(p, b, q, n);
+  const ll n3 = n3of(b), x = i3(b, i, j, k);
+  const double rho = qb[x], pp = qb[x + 4 * n3];
+  unsigned long long kind = 0;
+  if (pp <= p.qmin5) kind = 1;
+  else if (rho <= p.qmin1) kind = 2;
+  if (!kind) return;
+  const int im = b.imax - 1, jm = b.jmax - 1;
+  int reg, loc;
+  if (j >= 1 && j <= jm && k >= 1 && k <= b.kmax - 1) {
+    reg = 0;
+    loc = (i + 1) + (b.imax + 3) * ((j - 1) + jm * (k - 1));
+  } else if (j < 1 || j > jm) {
+    reg = j < 1 ? 1 : 2;
+    loc = (i - 1) + im * ((j < 1 ? j + 1 : j - b.jmax) + 2 * (k - 1));
+  } else {
+    reg = k < 1 ? 3 : 4;
+    loc = (i - 1) + im * ((j - 1) + jm * (k < 1 ? k + 1 : k - b.kmax));
+  }
+  atomicMin(flag, prtest_key(p, block, n, reg, loc, kind, stage_seq));
+}
+
+// The halo fill of a stage in one launch: BC patches, cut copies and, check
+// set, bprtest of every cell they set and of the interior.  Patches and cuts
+// read interior cells only and set halo cells, each set by one of them (the
+// launcher's condition), so their order is free.  Each is bound by the latency
+// of one work-group's chain, so that three launches cost the sum of them and
+// one the longest; the cut copies have a thread for every snapshot (one thread
+// ran through all of them).  HB O-grid, 9 snapshots: cut + BC + test 33 + 21 +
+// 9 us at the mean of the levels -> 28; one block of 4096 cells
+// 7.8 + 2.9 (no cuts) -> 8.6.  Whole cycles of the 193-node O-grid 11.9 -> 10.4 ms.
+__global__ void __launch_bounds__(256) k_halo(Par p, const Blk* __restrict__ blks, const PatchRec* __restrict__ pr,
+                                              const Tile* __restrict__ ptiles, int npt,
+                                              const CutRec* __restrict__ cr, const Tile* __restrict__ ctiles, int nct,
+                                              const Tile* __restrict__ cells, double* __restrict__ q,
+                                              const double* __restrict__ si, const double* __restrict__ sj,
+                                              const double* __restrict__ sk, const double* __restrict__ dist,
+                                              const double* __restrict__ qfb, int check, int stage_seq,
+                                              unsigned long long* __restrict__ flag) {
+  const int wg = blockIdx.x;
+  if (wg >= npt + nct) {   // interior cells
+    const Tile t = cells[wg - npt - nct];
+    const Blk b = blks[t.block];
+    CellIdx c;
+    if (!cell_of(p, b, t.base + threadIdx.x, c)) return;
+    prtest_cell(p, b, t.block, c.n, c.i, c.j, c.k, q, stage_seq, flag);
+    return;
+  }
+  HaloCells h;
+  int block;
+  if (wg < npt) {
+    const Tile tl = ptiles[wg];
+    const PatchRec rec = pr[tl.block];
+    const int item = tl.base + threadIdx.x;
+    if (item >= rec.count * p.nsnap) return;
+    const int n = item / rec.count;
+    block = rec.block;
+    bc_point(p, rec, blks[block], n, item - n * rec.count, q, si, sj, sk, dist, qfb, h);
+  } else {
+    const Tile tl = ctiles[wg - npt];
+    const CutRec rec = cr[tl.block];
+    const int item = tl.base + threadIdx.x;
+    if (item >= rec.count * p.nsnap) return;
+    const int n = item / rec.count;
+    block = rec.b1;
+    cut_point(p, rec, blks[block], blks[rec.b2], n, item - n * rec.count, q, h);
+  }
+  if (!check) return;
+  const Blk b = blks[block];
+  for (int m = 0; m < 2; m++) prtest_cell(p, b, block, h.n, h.i[m], h.j[m], h.k[m], q, stage_seq, flag);
 }
 
 // ---- q_bedges / q_bcorns (src/flux.f90:3914-4263, 3156-3471) ----
@@ -1453,18 +1553,29 @@ hipError_t launch_bc(Solve& s, Level& L, double* q) {
   }
   return hipGetLastError();
 }
-hipError_t launch_cut(Solve& s, Level& L, double* q) {
+// cut copies of a P3 array with p.npde variables: every record at once, or in
+// order for blocks one cell thick (a record may read another's halos there)
+static hipError_t cut_all(Solve& s, Level& L, const Par& p, double* a) {
   const int nc = (int)L.hcut.size();
   if (!nc) return hipSuccess;
-  if (!L.thin) {
-    dim3 g((L.maxcut + TS - 1) / TS, nc);
-    hipLaunchKernelGGL(k_cut, g, dim3(TS), 0, s.stream, s.par, L.dblk, L.dcut, 0, q);
-  } else {
-    for (int ic = 0; ic < nc; ic++) {
-      dim3 g((L.hcut[ic].count + TS - 1) / TS, 1);
-      hipLaunchKernelGGL(k_cut, g, dim3(TS), 0, s.stream, s.par, L.dblk, L.dcut, ic, q);
-    }
+  for (int ic = 0; ic < (L.thin ? nc : 1); ic++) {
+    const int t0 = L.ctile_first[ic], nt = L.ctile_first[L.thin ? ic + 1 : nc] - t0;
+    if (nt) hipLaunchKernelGGL(k_cut, dim3(nt), dim3(TS), 0, s.stream, p, L.dblk, L.dcut, L.ctile + t0, a);
   }
+  return hipGetLastError();
+}
+hipError_t launch_cut(Solve& s, Level& L, double* q) { return cut_all(s, L, s.par, q); }
+hipError_t launch_halo(Solve& s, Level& L, double* q, bool check, int stage_seq) {
+  if (!L.halo_once) {
+    hipError_t e = launch_bc(s, L, q);
+    if (e == hipSuccess) e = launch_cut(s, L, q);
+    return e;
+  }
+  const int npt = L.ptile_first.back(), nct = L.ctile_first.back(), nt = npt + nct + (check ? L.ntile[TK_CELLS] : 0);
+  if (nt)
+    hipLaunchKernelGGL(k_halo, dim3(nt), dim3(TS), 0, s.stream, s.par, L.dblk, L.dpatch, L.ptile, npt, L.dcut, L.ctile,
+                       nct, L.tile[TK_CELLS], q, L.f[COSAHIP_SI], L.f[COSAHIP_SJ], L.f[COSAHIP_SK],
+                       L.f[COSAHIP_DIST], s.dqfst, check ? 1 : 0, stage_seq, s.dflag + (L.nl - 1));
   return hipGetLastError();
 }
 hipError_t launch_edges_corners(Solve& s, Level& L, double* q) {
@@ -1485,20 +1596,9 @@ hipError_t launch_edges(Solve& s, Level& L, double* q, float* q32) {
 }
 // cut copies of a P3 array with ncomp variables per snapshot (mut: 1)
 hipError_t launch_cut_ncomp(Solve& s, Level& L, double* a, int ncomp) {
-  const int nc = (int)L.hcut.size();
-  if (!nc) return hipSuccess;
   Par p = s.par;
   p.npde = ncomp;
-  if (!L.thin) {
-    dim3 g((L.maxcut + TS - 1) / TS, nc);
-    hipLaunchKernelGGL(k_cut, g, dim3(TS), 0, s.stream, p, L.dblk, L.dcut, 0, a);
-  } else {
-    for (int ic = 0; ic < nc; ic++) {
-      dim3 g((L.hcut[ic].count + TS - 1) / TS, 1);
-      hipLaunchKernelGGL(k_cut, g, dim3(TS), 0, s.stream, p, L.dblk, L.dcut, ic, a);
-    }
-  }
-  return hipGetLastError();
+  return cut_all(s, L, p, a);
 }
 // rest4_b (src/cosa.f90:3122-3164): rest1 of a scalar P3 field
 hipError_t launch_rest_scalar(Solve& s, Level& L1, Level& L2, const double* a1, double* a2) {

@@ -32,6 +32,9 @@ hipError_t launch_rms(Solve& s, Level& L, const double* res, const double* rhs, 
 hipError_t launch_prtest(Solve& s, Level& L, const double* q, int stage_seq);
 hipError_t launch_bc(Solve& s, Level& L, double* q);
 hipError_t launch_cut(Solve& s, Level& L, double* q);
+// launch_bc and launch_cut; check: and, where the level's halos allow one launch
+// (Level::halo_once), launch_prtest too
+hipError_t launch_halo(Solve& s, Level& L, double* q, bool check = false, int stage_seq = 0);
 hipError_t launch_edges_corners(Solve& s, Level& L, double* q);
 hipError_t launch_rest1(Solve& s, Level& L1, Level& L2, const double* q1, double* q2);
 hipError_t launch_rest2(Solve& s, Level& L1, Level& L2, double* rhs2, const double* res1);
