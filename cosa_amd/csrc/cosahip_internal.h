@@ -105,6 +105,7 @@ enum TileKind {
   TK_STRIP_J,     // strips of cirs_strip_w lines along j (W cells along i x the whole j-line, all variables)
   TK_STRIP_K,     // the same along k
   TK_T32,         // residual tiles of 32 x 7 cells x kseg-plane k segments (RESID_TILE32_W4, RESID_SVA32)
+  TK_CELLV,       // interior cells x variables, all snapshots in one item (HB source of 3, 5, 7, 9 snapshots)
   TK_NKIND
 };
 

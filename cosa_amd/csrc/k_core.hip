@@ -78,7 +78,43 @@ __device__ __forceinline__ const double* qblk(const Par& p, const Blk& b, const 
   return q + b.o3 * p.npde * p.nsnap + n3of(b) * (ll)p.npde * n;
 }
 
+// The passes over cells take the variable count NV as a template argument and
+// load every variable before the first store, so that a thread has all its
+// loads in flight instead of one behind the store before it.  They are bound
+// by bandwidth on large levels (about 5 TB/s); k-omega wing, 2.1 M cells:
+// cons2prim 80 -> 69 us, update 89 -> 88, sums of squares 65 -> 56; HB
+// O-grid, 1.3 M cells: sums 22 -> 14, cons2prim 33 -> 30.  VARS5OR7 starts the
+// form of the run's variable count.
+#define VARS5OR7(kernel, grid, ...)                                                     \
+  do {                                                                                  \
+    if (s.par.npde == 7) hipLaunchKernelGGL(kernel<7>, grid, dim3(TS), 0, s.stream, __VA_ARGS__); \
+    else hipLaunchKernelGGL(kernel<5>, grid, dim3(TS), 0, s.stream, __VA_ARGS__);       \
+  } while (0)
+template <int NV, typename T>
+__device__ __forceinline__ void load_vars(T (&v)[NV], const T* a, ll x, ll n3) {
+#pragma unroll
+  for (int m = 0; m < NV; m++) v[m] = a[x + m * n3];
+}
+template <int NV, typename T>
+__device__ __forceinline__ void store_vars(const T (&v)[NV], T* a, ll x, ll n3) {
+#pragma unroll
+  for (int m = 0; m < NV; m++) a[x + m * n3] = v[m];
+}
+// one state, conservative to primitive
+template <int NV>
+__device__ __forceinline__ void to_prim(const Par& p, double (&v)[NV]) {
+  const double rho = v[0], u = v[1] / rho, vv = v[2] / rho, w = v[3] / rho;
+#pragma unroll
+  for (int m = 5; m < NV; m++) v[m] = v[m] / rho;
+  const double tke = NV > 5 ? v[NV - 2] : 0.0;
+  v[1] = u;
+  v[2] = vv;
+  v[3] = w;
+  v[4] = (p.gamma - 1) * (v[4] - rho * (u * u + vv * vv + w * w) / 2 - rho * tke);
+}
+
 // ---- cons2prim_b (src/update.f90:2136-2188), interior ----
+template <int NV>
 __global__ void __launch_bounds__(256) k_cons2prim(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                    double* __restrict__ q, float* __restrict__ q32,
                                                    double* __restrict__ qold) {
@@ -88,28 +124,17 @@ __global__ void __launch_bounds__(256) k_cons2prim(Par p, const Blk* __restrict_
   if (!cell_of(p, b, t.base + threadIdx.x, c)) return;
   double* qb = qblk(p, b, q, c.n);
   const ll n3 = n3of(b), x = i3(b, c.i, c.j, c.k);
-  if (qold) {   // copy_array of the conservative state first (the RK stage's qold)
-    double* ob = qblk(p, b, qold, c.n);
-    for (int m = 0; m < p.npde; m++) ob[x + m * n3] = qb[x + m * n3];
-  }
-  double rho = qb[x];
-  double u = qb[x + n3] / rho, v = qb[x + 2 * n3] / rho, w = qb[x + 3 * n3] / rho;
-  for (int m = 5; m < p.npde; m++) qb[x + m * n3] = qb[x + m * n3] / rho;
-  double rhoe = qb[x + 4 * n3];
-  double tke = p.kom ? qb[x + 5 * n3] : 0.0;
-  qb[x + n3] = u;
-  qb[x + 2 * n3] = v;
-  qb[x + 3 * n3] = w;
-  const double pp = (p.gamma - 1) * (rhoe - rho * (u * u + v * v + w * w) / 2 - rho * tke);
-  qb[x + 4 * n3] = pp;
+  double v[NV];
+  load_vars(v, qb, x, n3);
+  // copy_array of the conservative state first (the RK stage's qold)
+  if (qold) store_vars(v, qblk(p, b, qold, c.n), x, n3);
+  to_prim(p, v);
+#pragma unroll
+  for (int m = 1; m < NV; m++) qb[x + m * n3] = v[m];
   if (q32) {   // FP32 shadow of the primitive state for the FP32-residual mode
     float* sb = q32 + (qb - q);
-    sb[x] = (float)rho;
-    sb[x + n3] = (float)u;
-    sb[x + 2 * n3] = (float)v;
-    sb[x + 3 * n3] = (float)w;
-    sb[x + 4 * n3] = (float)pp;
-    for (int m = 5; m < p.npde; m++) sb[x + m * n3] = (float)qb[x + m * n3];
+#pragma unroll
+    for (int m = 0; m < NV; m++) sb[x + m * n3] = (float)v[m];
   }
 }
 
@@ -133,6 +158,7 @@ __global__ void __launch_bounds__(256) k_to_f32(const double* __restrict__ src, 
 }
 
 // ---- prim2cons_b (src/update.f90:1875-2084), interior + face halo strips ----
+template <int NV>
 __global__ void __launch_bounds__(256) k_prim2cons(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                    double* __restrict__ q, int halo_only) {
   const Tile t = tiles[blockIdx.x];
@@ -142,11 +168,13 @@ __global__ void __launch_bounds__(256) k_prim2cons(Par p, const Blk* __restrict_
   if (halo_only && reg == 0 && i >= 1 && i <= b.imax - 1) return;   // interior cell
   double* qb = qblk(p, b, q, n);
   const ll n3 = n3of(b), x = i3(b, i, j, k);
-  double rho = qb[x];
-  double rhou = qb[x + n3] * rho, rhov = qb[x + 2 * n3] * rho, rhow = qb[x + 3 * n3] * rho;
-  double tke = p.kom ? qb[x + 5 * n3] : 0.0;   // k saved before the scaling (work(:,1) of prim2cons_b)
-  for (int m = 5; m < p.npde; m++) qb[x + m * n3] = qb[x + m * n3] * rho;
-  double pp = qb[x + 4 * n3];
+  double v[NV];
+  load_vars(v, qb, x, n3);
+  const double rho = v[0], pp = v[4];
+  const double rhou = v[1] * rho, rhov = v[2] * rho, rhow = v[3] * rho;
+  const double tke = NV > 5 ? v[NV - 2] : 0.0;   // k before the scaling (work(:,1) of prim2cons_b)
+#pragma unroll
+  for (int m = 5; m < NV; m++) qb[x + m * n3] = v[m] * rho;
   qb[x + n3] = rhou;
   qb[x + 2 * n3] = rhov;
   qb[x + 3 * n3] = rhow;
@@ -154,6 +182,7 @@ __global__ void __launch_bounds__(256) k_prim2cons(Par p, const Blk* __restrict_
 }
 
 // ---- copy_array / add_array, off_l = -1 (src/util.f90:2-236) ----
+template <int NV>
 __global__ void __launch_bounds__(256) k_copy_int(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                   double* __restrict__ dst, const double* __restrict__ src) {
   const Tile t = tiles[blockIdx.x];
@@ -163,8 +192,11 @@ __global__ void __launch_bounds__(256) k_copy_int(Par p, const Blk* __restrict__
   const ll n3 = n3of(b), x = i3(b, c.i, c.j, c.k);
   double* d = qblk(p, b, dst, c.n);
   const double* s = qblk(p, b, src, c.n);
-  for (int v = 0; v < p.npde; v++) d[x + v * n3] = s[x + v * n3];
+  double v[NV];
+  load_vars(v, s, x, n3);
+  store_vars(v, d, x, n3);
 }
+template <int NV>
 __global__ void __launch_bounds__(256) k_add_int(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                  double* __restrict__ dst, const double* __restrict__ src,
                                                  double fact) {
@@ -175,7 +207,11 @@ __global__ void __launch_bounds__(256) k_add_int(Par p, const Blk* __restrict__ 
   const ll n3 = n3of(b), x = i3(b, c.i, c.j, c.k);
   double* d = qblk(p, b, dst, c.n);
   const double* s = qblk(p, b, src, c.n);
-  for (int v = 0; v < p.npde; v++) d[x + v * n3] = d[x + v * n3] + s[x + v * n3] * fact;
+  double v[NV], a[NV];
+  load_vars(v, d, x, n3);
+  load_vars(a, s, x, n3);
+#pragma unroll
+  for (int m = 0; m < NV; m++) d[x + m * n3] = v[m] + a[m] * fact;
 }
 
 // ---- zero (src/util.f90:238-369) on 0..imax x 0..jmax x 0..kmax ----
@@ -238,6 +274,7 @@ __global__ void __launch_bounds__(256) k_zero_shell(Par p, const Blk* __restrict
 }
 
 // q2 = q2 + qold2 * (-1) on 0..imax (add_array off_l = 1, prolong)
+template <int NV>
 __global__ void __launch_bounds__(256) k_sub_box(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                  double* __restrict__ dst, const double* __restrict__ src) {
   const Tile t = tiles[blockIdx.x];
@@ -253,13 +290,18 @@ __global__ void __launch_bounds__(256) k_sub_box(Par p, const Blk* __restrict__ 
   double* d = qblk(p, b, dst, n);
   const double* s = qblk(p, b, src, n);
   const ll n3 = n3of(b), y = i3(b, i, j, k);
-  for (int v = 0; v < p.npde; v++) d[y + v * n3] = d[y + v * n3] + s[y + v * n3] * -1.0;
+  double v[NV], a[NV];
+  load_vars(v, d, y, n3);
+  load_vars(a, s, y, n3);
+#pragma unroll
+  for (int m = 0; m < NV; m++) d[y + m * n3] = v[m] + a[m] * -1.0;
 }
 
 // ---- update_b / update_bhb explicit (src/update.f90:568-624, 1359-1408) ----
 // With Wilcox k-omega: the point-implicit rho*omega, rho*k update first
 // (src/update.f90:596-634), reading rho, k, omega of the current state;
 // ttrm(:,2:3) of kom are the constants gkw, bkw.
+template <int NV>
 __global__ void __launch_bounds__(256) k_update(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                 const double* __restrict__ res, double* __restrict__ q,
                                                 const double* __restrict__ qold, const double* __restrict__ dtvol,
@@ -276,28 +318,30 @@ __global__ void __launch_bounds__(256) k_update(Par p, const Blk* __restrict__ b
   double* qb = qblk(p, b, q, c.n);
   const double* ob = qblk(p, b, qold, c.n);
   const double* rb = qblk(p, b, res, c.n);
-  if (p.kom) {
-    const double rho = qb[x];
-    const double ome = qb[x + 6 * n3] / qb[x];
-    const double tke = qb[x + 5 * n3] / qb[x];
-    const double dtt = dtvolt[po];
-    const double dtau = dtt * vol[b.o1 + i1(b, c.i, c.j, c.k)];
+  double o[NV], r[NV];
+  load_vars(o, ob, x, n3);
+  load_vars(r, rb, x, n3);
+  if constexpr (NV > 5) {
+    const double rho = qb[x], rhok = qb[x + 5 * n3], rhoo = qb[x + 6 * n3];
+    const double dtt = dtvolt[po], vc = vol[b.o1 + i1(b, c.i, c.j, c.k)];
     const ll so = b.o3 * p.nsnap + n3 * (ll)c.n + x;
     // ttrm(2:3): the constants gkw, bkw of Wilcox k-omega, blended for BSL/SST
     const double* tb = p.sst ? ttrm + b.o3 * 3 * p.nsnap + n3 * 3 * (ll)c.n + x : nullptr;
     const double gav = tb ? tb[n3] : p.gkw, bav = tb ? tb[2 * n3] : p.bkw;
-    const double dl = delpls[so];
-    double rhomega = (ob[x + 6 * n3] - ar * rb[x + 6 * n3] * dtt + ar * dtau * rho * ome * (gav * dl + 2 * bav * ome)) /
+    const double dl = delpls[so], pr = prd[so];
+    const double ome = rhoo / rho, tke = rhok / rho, dtau = dtt * vc;
+    double rhomega = (o[6] - ar * r[6] * dtt + ar * dtau * rho * ome * (gav * dl + 2 * bav * ome)) /
                      (1 + ar * dtau * (gav * dl + 2 * bav * ome));
-    const double rhomegamin = gav * p.cmu * rho * sqrt(prd[so]);
+    const double rhomegamin = gav * p.cmu * rho * sqrt(pr);
     if (rhomega < rhomegamin) rhomega = rhomegamin;
     qb[x + 6 * n3] = rhomega;
     const double drhomega = rhomega - rho * ome;
-    qb[x + 5 * n3] = (ob[x + 5 * n3] - ar * rb[x + 5 * n3] * dtt + ar * dtau * rho * tke * (dl + p.bstrkw * ome) -
+    qb[x + 5 * n3] = (o[5] - ar * r[5] * dtt + ar * dtau * rho * tke * (dl + p.bstrkw * ome) -
                       ar * dtau * p.bstrkw * tke * drhomega) /
                      (1 + ar * dtau * (dl + p.bstrkw * ome));
   }
-  for (int v = 0; v < 5; v++) qb[x + v * n3] = ob[x + v * n3] - ar * rb[x + v * n3] * dt;
+#pragma unroll
+  for (int v = 0; v < 5; v++) qb[x + v * n3] = o[v] - ar * r[v] * dt;
 }
 
 // ---- dual time stepping (one snapshot), interior cells ----------------------
@@ -463,6 +507,43 @@ __global__ void __launch_bounds__(256) k_src_hb(Par p, const Blk* __restrict__ b
     for (int nj = 0; nj < ns; nj++) acc = acc + p.omega * vv * dhb[ni + ns * nj] * qb[stride_n * nj + n3 * v];
     hb[stride_n * ni + n3 * v] = acc;
     rb[stride_n * ni + n3 * v] = rb[stride_n * ni + n3 * v] + acc;
+  }
+}
+
+// The same with a thread for a cell and variable of all NS snapshots: it loads
+// the NS states once, where a thread of k_src_hb loads them all for one
+// snapshot's source, NS times over, one variable after another.  For up to 4
+// harmonics (TK_CELLV); above, the unrolled NS x NS sums no longer fit the
+// registers.  147456 cells x 9
+// snapshots: 84 -> 39 us against k_src_hb (5.4 TB/s).
+template <int NS>
+__global__ void __launch_bounds__(256) k_src_hbv(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
+                                                 const double* __restrict__ q, const double* __restrict__ vol,
+                                                 double* __restrict__ res, double* __restrict__ qhb,
+                                                 const double* __restrict__ dhb) {
+  const Tile t = tiles[blockIdx.x];
+  const Blk b = blks[t.block];
+  const int im = b.imax - 1, jm = b.jmax - 1, nc = im * jm * (b.kmax - 1);
+  const int item = t.base + threadIdx.x;
+  if (item >= nc * p.npde) return;
+  const int v = item / nc;
+  int rem = item - v * nc;
+  const int i = rem % im + 1;
+  rem /= im;
+  const int j = rem % jm + 1, k = rem / jm + 1;
+  const ll n3 = n3of(b), stride_n = n3 * p.npde;
+  const ll x = b.o3 * p.npde * p.nsnap + n3 * v + i3(b, i, j, k);
+  const double vv = vol[b.o1 + i1(b, i, j, k)];
+  double s[NS], r[NS];
+  load_vars(s, q, x, stride_n);
+  load_vars(r, res, x, stride_n);
+#pragma unroll
+  for (int ni = 0; ni < NS; ni++) {
+    double acc = 0.0;
+#pragma unroll
+    for (int nj = 0; nj < NS; nj++) acc = acc + p.omega * vv * dhb[ni + NS * nj] * s[nj];
+    qhb[x + stride_n * ni] = acc;
+    res[x + stride_n * ni] = r[ni] + acc;
   }
 }
 
@@ -724,32 +805,38 @@ __global__ void __launch_bounds__(256) k_rms_hb_term(Par p, const Blk* __restric
 }
 
 // ---- resg_brms (src/cosa.f90:4503-4582): per-tile partial sums ----
+template <int NV>
 __global__ void __launch_bounds__(256) k_rms_part(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                   const double* __restrict__ res, const double* __restrict__ rhs,
                                                   int use_rhs, double* __restrict__ part) {
-  __shared__ double sh[7][256];
+  __shared__ double sh[NV][256];
   const Tile t = tiles[blockIdx.x];
   const Blk b = blks[t.block];
   CellIdx c;
-  double s[7] = {0, 0, 0, 0, 0, 0, 0};
-  const int nv = p.npde;
+  double s[NV] = {};
   if (cell_of(p, b, t.base + threadIdx.x, c)) {
     const ll n3 = n3of(b), x = i3(b, c.i, c.j, c.k);
     const double* rb = qblk(p, b, res, c.n);
-    const double* hb = use_rhs ? qblk(p, b, rhs, c.n) : nullptr;
-    for (int v = 0; v < nv; v++) {
-      double d = use_rhs ? rb[x + v * n3] - hb[x + v * n3] : rb[x + v * n3];
-      s[v] = d * d;
+    load_vars(s, rb, x, n3);
+    if (use_rhs) {
+      double h[NV];
+      load_vars(h, qblk(p, b, rhs, c.n), x, n3);
+#pragma unroll
+      for (int v = 0; v < NV; v++) s[v] = s[v] - h[v];
     }
+#pragma unroll
+    for (int v = 0; v < NV; v++) s[v] = s[v] * s[v];
   }
-  for (int v = 0; v < nv; v++) sh[v][threadIdx.x] = s[v];
+#pragma unroll
+  for (int v = 0; v < NV; v++) sh[v][threadIdx.x] = s[v];
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w)
-      for (int v = 0; v < nv; v++) sh[v][threadIdx.x] += sh[v][threadIdx.x + w];
+#pragma unroll
+      for (int v = 0; v < NV; v++) sh[v][threadIdx.x] += sh[v][threadIdx.x + w];
     __syncthreads();
   }
-  if ((int)threadIdx.x < nv) part[(ll)blockIdx.x * 8 + threadIdx.x] = sh[threadIdx.x][0];
+  if ((int)threadIdx.x < NV) part[(ll)blockIdx.x * 8 + threadIdx.x] = sh[threadIdx.x][0];
 }
 // fixed-order final reduction: one workgroup, strided partial sums then tree
 __global__ void __launch_bounds__(256) k_rms_final(const double* __restrict__ part, int nt, int nv,
@@ -1384,7 +1471,7 @@ __global__ void __launch_bounds__(256) k_prol(Par p, const Blk* __restrict__ b1s
 hipError_t launch_cons2prim(Solve& s, Level& L, double* q, bool shadow, double* qold) {
   float* q32 = shadow && s.fp32() && q == L.f[COSAHIP_Q] ? L.q32 : nullptr;
   if (L.ntile[TK_CELLS])
-    hipLaunchKernelGGL(k_cons2prim, grid1(L.ntile[TK_CELLS]), dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLS], q,
+    VARS5OR7(k_cons2prim, grid1(L.ntile[TK_CELLS]), s.par, L.dblk, L.tile[TK_CELLS], q,
                        q32, qold);
   return hipGetLastError();
 }
@@ -1403,19 +1490,19 @@ hipError_t launch_to_f32(Solve& s, const double* src, float* dst, ll n) {
 }
 hipError_t launch_prim2cons(Solve& s, Level& L, double* q, bool halo_only) {
   if (L.ntile[TK_HALO])
-    hipLaunchKernelGGL(k_prim2cons, grid1(L.ntile[TK_HALO]), dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_HALO], q,
+    VARS5OR7(k_prim2cons, grid1(L.ntile[TK_HALO]), s.par, L.dblk, L.tile[TK_HALO], q,
                        halo_only ? 1 : 0);
   return hipGetLastError();
 }
 hipError_t launch_copy_interior(Solve& s, Level& L, double* dst, const double* src) {
   if (L.ntile[TK_CELLS])
-    hipLaunchKernelGGL(k_copy_int, grid1(L.ntile[TK_CELLS]), dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLS],
+    VARS5OR7(k_copy_int, grid1(L.ntile[TK_CELLS]), s.par, L.dblk, L.tile[TK_CELLS],
                        dst, src);
   return hipGetLastError();
 }
 hipError_t launch_add_interior(Solve& s, Level& L, double* dst, const double* src, double fact) {
   if (L.ntile[TK_CELLS])
-    hipLaunchKernelGGL(k_add_int, grid1(L.ntile[TK_CELLS]), dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLS],
+    VARS5OR7(k_add_int, grid1(L.ntile[TK_CELLS]), s.par, L.dblk, L.tile[TK_CELLS],
                        dst, src, fact);
   return hipGetLastError();
 }
@@ -1433,7 +1520,7 @@ hipError_t launch_zero_res_shell(Solve& s, Level& L, double* res) {
 }
 hipError_t launch_sub_box(Solve& s, Level& L, double* dst, const double* src) {
   if (L.ntile[TK_CELLS_P1])
-    hipLaunchKernelGGL(k_sub_box, grid1(L.ntile[TK_CELLS_P1]), dim3(TS), 0, s.stream, s.par, L.dblk,
+    VARS5OR7(k_sub_box, grid1(L.ntile[TK_CELLS_P1]), s.par, L.dblk,
                        L.tile[TK_CELLS_P1], dst, src);
   return hipGetLastError();
 }
@@ -1504,23 +1591,34 @@ hipError_t launch_update(Solve& s, Level& L, double ar) {
     return hipGetLastError();
   }
   if (L.ntile[TK_CELLS])
-    hipLaunchKernelGGL(k_update, grid1(L.ntile[TK_CELLS]), dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLS],
+    VARS5OR7(k_update, grid1(L.ntile[TK_CELLS]), s.par, L.dblk, L.tile[TK_CELLS],
                        L.f[COSAHIP_RES], L.f[COSAHIP_Q], L.f[COSAHIP_QOLD], L.f[COSAHIP_DTVOL], ar,
                        L.f[COSAHIP_VOL], L.f[COSAHIP_DTVOLT], L.f[COSAHIP_DELPLS], L.f[COSAHIP_PRD],
                        L.f[COSAHIP_TTRM]);
   return hipGetLastError();
 }
 hipError_t launch_src_hb(Solve& s, Level& L) {
-  // one work item per interior (cell, snapshot)
-  if (L.ntile[TK_CELLS])
+  if (L.ntile[TK_CELLV]) {
+    const dim3 g = grid1(L.ntile[TK_CELLV]);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, g, dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLV], L.f[COSAHIP_Q],
+                         L.f[COSAHIP_VOL], L.f[COSAHIP_RES], L.dq, s.ddhb);
+    };
+    if (s.par.nsnap == 3) go(k_src_hbv<3>);
+    else if (s.par.nsnap == 5) go(k_src_hbv<5>);
+    else if (s.par.nsnap == 7) go(k_src_hbv<7>);
+    else go(k_src_hbv<9>);
+  } else if (L.ntile[TK_CELLS]) {
+    // one work item per interior (cell, snapshot)
     hipLaunchKernelGGL(k_src_hb, grid1(L.ntile[TK_CELLS]), dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLS],
                        L.f[COSAHIP_Q], L.f[COSAHIP_VOL], L.f[COSAHIP_RES], L.dq, s.ddhb);
+  }
   return hipGetLastError();
 }
 hipError_t launch_rms(Solve& s, Level& L, const double* res, const double* rhs, int use_rhs) {
   const int nt = L.ntile[TK_CELLS];
   if (!nt) return hipSuccess;
-  hipLaunchKernelGGL(k_rms_part, grid1(nt), dim3(256), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLS], res, rhs,
+  VARS5OR7(k_rms_part, grid1(nt), s.par, L.dblk, L.tile[TK_CELLS], res, rhs,
                      use_rhs, L.rms_part);
   hipLaunchKernelGGL(k_rms_final, dim3(1), dim3(256), 0, s.stream, L.rms_part, nt, s.par.npde,
                      L.rms_part + (ll)nt * 8);
