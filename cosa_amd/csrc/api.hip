@@ -2019,6 +2019,9 @@ static int smooth_core(Solve* s, int nl, int from_fine, int to_coarse, int niter
   // stage's cons2prim (mean flow with cirs: the state is the same bits)
   const bool fuse_update = s->fuse_update && !komega(c) && s->par.irsop >= 1 && s->par.irsop != 4 &&
                            s->par.irsop <= 6 && c.cutcirs != 1 && !c.rkimp;
+  // otherwise fixq and the next stage's cons2prim go into the update, where
+  // it has a form that does them (q is not conservative between the stages)
+  const bool tail = !fuse_update && s->fuse_update && update_takes_tail(*s);
   bool q_prim = false;   // the previous stage left q in primitive variables
   for (int iter = 1; iter <= niterp && !returned_early; iter++) {
     const ll cs = L.ncell * s->par.nsnap;
@@ -2128,14 +2131,19 @@ static int smooth_core(Solve* s, int nl, int from_fine, int to_coarse, int niter
           TimeScope t(*s, COSAHIP_FAM_CIRS, cs);
           CK(launch_cirs(*s, L));
         }
-        {
-          TimeScope t(*s, COSAHIP_FAM_UPDATE, cs);
-          CK(launch_update(*s, L, c.alphas[irk - 1]));
+        UpdateTail up;
+        if (tail) {
+          up.fix = komega(c) && c.ifixq == 1;
+          up.prim = irk < c.nstage;
+          up.q32 = up.prim && s->fp32() ? L.q32 : nullptr;
+          q_prim = up.prim != 0;
         }
+        TimeScope t(*s, COSAHIP_FAM_UPDATE, cs);
+        CK(launch_update(*s, L, c.alphas[irk - 1], up));
       }
       if (komega(c)) {
         TimeScope t(*s, COSAHIP_FAM_OTHER, cs);
-        if (c.ifixq == 1) CK(launch_fixq(*s, L));
+        if (c.ifixq == 1 && !tail) CK(launch_fixq(*s, L));
         if (irk == c.nstage && (nl == 1 || !c.prd_all_lvls)) CK(launch_tur_vis(*s, L, q));
       }
     }

@@ -293,7 +293,7 @@ struct Solve {
   Par par;
   int device = 0;
   double* scratch = nullptr;   // this GPU's fixed force scratch array (cosahip_force_noalloc)
-  bool fuse_update = true;     // RK update and next cons2prim in the last CIRS sweep (COSAHIP_FUSED_UPDATE=0: off)
+  bool fuse_update = true;     // RK update and next cons2prim in the last CIRS sweep, or cons2prim (and fixq) in the update (COSAHIP_FUSED_UPDATE=0: off)
   hipStream_t stream = nullptr;
   std::vector<Level> lev;     // index nl-1
   double dhb[131 * 131];      // dhb(i,j) column-major

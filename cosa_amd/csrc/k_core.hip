@@ -301,13 +301,19 @@ __global__ void __launch_bounds__(256) k_sub_box(Par p, const Blk* __restrict__ 
 // With Wilcox k-omega: the point-implicit rho*omega, rho*k update first
 // (src/update.f90:596-634), reading rho, k, omega of the current state;
 // ttrm(:,2:3) of kom are the constants gkw, bkw.
+// up.fix: fixq_b of the new state in the same pass; up.prim: the state left
+// primitive (with its FP32 shadow up.q32), as the next stage's cons2prim would
+// make it.  The pass is bound by bandwidth, and the two that followed it read
+// and wrote what it had in registers: k-omega wing, 2.1 M cells, update + fixq
+// + cons2prim 88 + 12 + 69 us in three passes.
 template <int NV>
 __global__ void __launch_bounds__(256) k_update(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
                                                 const double* __restrict__ res, double* __restrict__ q,
                                                 const double* __restrict__ qold, const double* __restrict__ dtvol,
                                                 double ar, const double* __restrict__ vol,
                                                 const double* __restrict__ dtvolt, const double* __restrict__ delpls,
-                                                const double* __restrict__ prd, const double* __restrict__ ttrm) {
+                                                const double* __restrict__ prd, const double* __restrict__ ttrm,
+                                                UpdateTail up) {
   const Tile t = tiles[blockIdx.x];
   const Blk b = blks[t.block];
   CellIdx c;
@@ -318,7 +324,7 @@ __global__ void __launch_bounds__(256) k_update(Par p, const Blk* __restrict__ b
   double* qb = qblk(p, b, q, c.n);
   const double* ob = qblk(p, b, qold, c.n);
   const double* rb = qblk(p, b, res, c.n);
-  double o[NV], r[NV];
+  double o[NV], r[NV], w[NV];
   load_vars(o, ob, x, n3);
   load_vars(r, rb, x, n3);
   if constexpr (NV > 5) {
@@ -334,14 +340,27 @@ __global__ void __launch_bounds__(256) k_update(Par p, const Blk* __restrict__ b
                      (1 + ar * dtau * (gav * dl + 2 * bav * ome));
     const double rhomegamin = gav * p.cmu * rho * sqrt(pr);
     if (rhomega < rhomegamin) rhomega = rhomegamin;
-    qb[x + 6 * n3] = rhomega;
+    w[6] = rhomega;
     const double drhomega = rhomega - rho * ome;
-    qb[x + 5 * n3] = (o[5] - ar * r[5] * dtt + ar * dtau * rho * tke * (dl + p.bstrkw * ome) -
+    w[5] = (o[5] - ar * r[5] * dtt + ar * dtau * rho * tke * (dl + p.bstrkw * ome) -
                       ar * dtau * p.bstrkw * tke * drhomega) /
-                     (1 + ar * dtau * (dl + p.bstrkw * ome));
+           (1 + ar * dtau * (dl + p.bstrkw * ome));
   }
 #pragma unroll
-  for (int v = 0; v < 5; v++) qb[x + v * n3] = o[v] - ar * r[v] * dt;
+  for (int v = 0; v < 5; v++) w[v] = o[v] - ar * r[v] * dt;
+  if constexpr (NV > 5) {
+    if (up.fix) {
+      if (w[5] / w[0] < p.qmin6) w[5] = w[0] * p.qmin6;
+      if (w[6] / w[0] < p.qmin7) w[6] = w[0] * p.qmin7;
+    }
+  }
+  if (up.prim) to_prim(p, w);
+  store_vars(w, qb, x, n3);
+  if (up.q32) {
+    float* sb = up.q32 + (qb - q);
+#pragma unroll
+    for (int m = 0; m < NV; m++) sb[x + m * n3] = (float)w[m];
+  }
 }
 
 // ---- dual time stepping (one snapshot), interior cells ----------------------
@@ -1580,7 +1599,8 @@ hipError_t launch_rms_dual_term(Solve& s, Level& L, double* work1) {
                        work1);
   return hipGetLastError();
 }
-hipError_t launch_update(Solve& s, Level& L, double ar) {
+bool update_takes_tail(const Solve& s) { return !(s.cfg.harbal && s.cfg.rkimp) && !s.par.dual_rkimp; }
+hipError_t launch_update(Solve& s, Level& L, double ar, const UpdateTail& up) {
   if (s.cfg.harbal && s.cfg.rkimp) return launch_update_rkim(s, L, ar);
   if (s.par.dual_rkimp) {
     if (L.ntile[TK_CELLS])
@@ -1594,7 +1614,7 @@ hipError_t launch_update(Solve& s, Level& L, double ar) {
     VARS5OR7(k_update, grid1(L.ntile[TK_CELLS]), s.par, L.dblk, L.tile[TK_CELLS],
                        L.f[COSAHIP_RES], L.f[COSAHIP_Q], L.f[COSAHIP_QOLD], L.f[COSAHIP_DTVOL], ar,
                        L.f[COSAHIP_VOL], L.f[COSAHIP_DTVOLT], L.f[COSAHIP_DELPLS], L.f[COSAHIP_PRD],
-                       L.f[COSAHIP_TTRM]);
+                       L.f[COSAHIP_TTRM], up);
   return hipGetLastError();
 }
 hipError_t launch_src_hb(Solve& s, Level& L) {

@@ -18,7 +18,15 @@ hipError_t launch_copy_interior(Solve& s, Level& L, double* dst, const double* s
 hipError_t launch_add_interior(Solve& s, Level& L, double* dst, const double* src, double fact);
 hipError_t launch_zero_res(Solve& s, Level& L, double* res);        // 0..imax box
 hipError_t launch_zero_res_shell(Solve& s, Level& L, double* res);  // first halo layer only
-hipError_t launch_update(Solve& s, Level& L, double ar);
+// What the update pass does to the new state besides storing it (forms of the
+// update that take it: update_takes_tail): fix: k-omega's fixq; prim: left in
+// primitive variables, with their FP32 shadow q32 (or null)
+struct UpdateTail {
+  int fix = 0, prim = 0;
+  float* q32 = nullptr;
+};
+bool update_takes_tail(const Solve& s);
+hipError_t launch_update(Solve& s, Level& L, double ar, const UpdateTail& up = {});
 int rkim_group(int m);
 hipError_t launch_lim_res_ome_rkim(Solve& s, Level& L);
 hipError_t launch_rms_hb_term(Solve& s, Level& L, double* work1);
