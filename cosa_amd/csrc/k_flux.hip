@@ -1047,7 +1047,9 @@ __device__ __forceinline__ void strip_forward(double* __restrict__ x, const doub
 }
 // Forward, coefficients eps(a) at g[a W]; store: keep the multipliers r(a)
 // at r[a W] for every line of the group.  (At a = 0 tridi's a is 0, here
-// t(-1) = r(-1) = -0 take its place.)
+// t(-1) = r(-1) = -0 take its place.)  The chain d(a) -> r(a) bounds it, so the
+// two quotients by d(a) share its inverse (Divisor, the bits of the division).
+// SST O-grid, i-lines of 256 cells: 55 -> 40 us, j-lines of 64 18.8 -> 16.9.
 template <int U>
 __device__ __forceinline__ void strip_forward_v_run(double* __restrict__ x, const double* __restrict__ g,
                                                     double* __restrict__ r, int a0, int L, int W, bool store,
@@ -1061,9 +1063,9 @@ __device__ __forceinline__ void strip_forward_v_run(double* __restrict__ x, cons
 #pragma unroll
   for (int u = 0; u < U; u++) {
     const double ca = -ev[u], cb = 1 + 2 * ev[u], cc = a0 + u == L - 1 ? 0.0 : -ev[u];
-    const double d = cb - rp * ca;
-    xv[u] = tp = (xv[u] - tp * ca) / d;
-    ev[u] = rp = cc / d;
+    const Divisor<double> d(cb - rp * ca);
+    xv[u] = tp = d.of(xv[u] - tp * ca);
+    ev[u] = rp = d.of(cc);
   }
 #pragma unroll
   for (int u = 0; u < U; u++) {
