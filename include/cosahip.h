@@ -473,7 +473,7 @@ enum {
   COSAHIP_FAM_RESIDUAL = 0,  /* MUSCL + Roe + flux difference, 3 directions */
   COSAHIP_FAM_CIRS = 1,      /* implicit residual smoothing, 3 sweeps       */
   COSAHIP_FAM_UPDATE = 2,    /* RK update                                   */
-  COSAHIP_FAM_HALO = 3,      /* BC patches and cut copies                   */
+  COSAHIP_FAM_HALO = 3,      /* BC patches, cut copies and (one launch) check */
   COSAHIP_FAM_CONVERT = 4,   /* cons2prim / prim2cons                       */
   COSAHIP_FAM_LAMBDA = 5,    /* spectral radii + local time step            */
   COSAHIP_FAM_OTHER = 6,     /* copies, FAS, norms, HB, MG transfer, checks */
