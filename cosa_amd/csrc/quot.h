@@ -90,8 +90,9 @@ __device__ __forceinline__ T face_sqrt(T x, T& rs) {
 // library's pow is within one -- in a dozen instructions instead of some two
 // hundred.  0 gives 0, a negative t NaN, as pow does.
 // k-omega wing, level 1 (2.1 M cells): the spectral radii, seven of these a
-// cell, 224 -> 149 us (105 since the smoothing's powers are out of their kernel); the viscous faces, with the quotients of viscous_face,
-// 209/204/192 -> 202/196/184 us -- they are bound by their loads.
+// cell, 224 -> 149 us (105 since the smoothing's powers are out of their
+// kernel); the viscous faces, with the quotients of viscous_face, 209/204/192
+// -> 202/196/184 us -- they are bound by their loads.
 template <typename T>
 __device__ __forceinline__ T pow32(T t) {
   const T s = sqrt(t);
