@@ -595,50 +595,57 @@ static bool cut_in_bounds(const Blk& b1, const Blk& b2, const int32_t* t, int n2
 
 static ll field_size(const Solve* s, const Level& L, int field);
 
-// Every face-halo cell of every block is set by exactly one point of one patch
-// or cut, and no block is one cell thick: then the halo fill and bprtest may
-// run as one launch (k_halo) -- no order between patches and cuts matters, and
-// the cells they set are all the halo cells bprtest looks at.
-static bool halos_set_once(const Level& L) {
-  if (L.thin) return false;
+// What the halo fill of a level may be relied on for.
+// halo_fresh: every face-halo cell of every block is set by each fill, from
+// interior cells alone.  A wall, symmetry or cut record reads two cells deep,
+// so in a block one cell thick it reads the far halo; a face that no record
+// covers keeps what it holds.
+// halo_once: besides, each is set by exactly one point of one patch or cut, and
+// no block is one cell thick: then the halo fill and bprtest may run as one
+// launch (k_halo) -- no order between patches and cuts matters, and the cells
+// they set are all the halo cells bprtest looks at.
+static void plan_halos(Level& L) {
   std::vector<std::vector<unsigned char>> hit(6 * (size_t)L.nblocks);
+  bool fresh = true, once = !L.thin;
+  auto ext = [&](int b, int d) {
+    const Blk& B = L.hblk[b];
+    return (d == 1 ? B.imax : d == 2 ? B.jmax : B.kmax) - 1;
+  };
   auto mark = [&](int block, int idir, int inout, int c2lo, int c2hi, int c3lo, int c3hi) {
     // transverse extents in the cyclic order of the record
-    const Blk& B = L.hblk[block];
-    const int ext[4] = {0, B.imax - 1, B.jmax - 1, B.kmax - 1};
-    const int e2 = ext[idir % 3 + 1], e3 = ext[(idir + 1) % 3 + 1];
+    const int e2 = ext(block, idir % 3 + 1), e3 = ext(block, (idir + 1) % 3 + 1);
     auto& h = hit[6 * (size_t)block + 2 * (idir - 1) + (inout == 1 ? 0 : 1)];
     if (h.empty()) h.assign((size_t)e2 * e3, 0);
-    if (c2lo < 1 || c3lo < 1 || c2hi > e2 || c3hi > e3) return false;
-    for (int c3 = c3lo; c3 <= c3hi; c3++)
-      for (int c2 = c2lo; c2 <= c2hi; c2++)
-        if (h[(size_t)(c3 - 1) * e2 + c2 - 1]++) return false;
-    return true;
+    if (c2lo < 1 || c3lo < 1 || c2hi > e2 || c3hi > e3) once = false;
+    for (int c3 = std::max(c3lo, 1); c3 <= std::min(c3hi, e3); c3++)
+      for (int c2 = std::max(c2lo, 1); c2 <= std::min(c2hi, e2); c2++) {
+        unsigned char& c = h[(size_t)(c3 - 1) * e2 + c2 - 1];
+        if (c) once = false;
+        c = 1;
+      }
   };
   for (const PatchRec& r : L.hpatch) {
     const int i2 = r.t[1] % 3 + 1, i3 = (r.t[1] + 1) % 3 + 1;
-    if (!mark(r.block, r.t[1], r.t[2], r.t[2 * i2 + 1], r.t[2 * i2 + 2], r.t[2 * i3 + 1], r.t[2 * i3 + 2])) return false;
+    mark(r.block, r.t[1], r.t[2], r.t[2 * i2 + 1], r.t[2 * i2 + 2], r.t[2 * i3 + 1], r.t[2 * i3 + 2]);
+    if (r.type != 30 && r.type != 4 && ext(r.block, r.t[1]) < 2) fresh = false;
   }
   for (const CutRec& r : L.hcut) {
     const int i2 = r.t[1] % 3 + 1, i3 = (r.t[1] + 1) % 3 + 1;
     const int a2 = r.t[2 * i2 + 1], b2 = r.t[2 * i2 + 2], a3 = r.t[2 * i3 + 1], b3 = r.t[2 * i3 + 2];
-    if (!mark(r.b1, r.t[1], r.t[2], std::min(a2, b2), std::max(a2, b2), std::min(a3, b3), std::max(a3, b3))) return false;
+    mark(r.b1, r.t[1], r.t[2], std::min(a2, b2), std::max(a2, b2), std::min(a3, b3), std::max(a3, b3));
     // the sources: interior cells of block 2 (cut_in_bounds allows its halos)
-    const Blk& B2 = L.hblk[r.b2];
-    const int ext[4] = {0, B2.imax - 1, B2.jmax - 1, B2.kmax - 1};
+    if (ext(r.b2, r.t[10]) < 2) fresh = false;
     for (int m = 1; m <= 2; m++) {
       const int d = r.t[17 + (r.t[1] + m - 1) % 3 + 1], len = m == 1 ? b2 - a2 : b3 - a3;
       const int lo = r.t[10 + 2 * d], sg = r.t[11 + 2 * d] > lo ? 1 : -1;
       const int hi = lo + sg * std::abs(len);
-      if (std::min(lo, hi) < 1 || std::max(lo, hi) > ext[d]) return false;
+      if (std::min(lo, hi) < 1 || std::max(lo, hi) > ext(r.b2, d)) fresh = false;
     }
   }
-  for (const auto& h : hit) {
-    if (h.empty()) return false;
-    for (unsigned char c : h)
-      if (c != 1) return false;
-  }
-  return true;
+  for (const auto& h : hit)
+    if (h.empty() || std::find(h.begin(), h.end(), 0) != h.end()) fresh = false;
+  L.halo_fresh = fresh;
+  L.halo_once = fresh && once;
 }
 
 // FP32 shadows of the level's primitive q and face metrics (FP32-residual mode)
@@ -852,7 +859,7 @@ extern "C" int cosahip_define_level(cosahip_solve* h, int nl, int nblocks, const
     L.ctile_first.push_back((int)L.hctile.size());
   }
   CK(upload_vec(&L.ctile, L.hctile));
-  L.halo_once = halos_set_once(L);
+  plan_halos(L);
   CK(upload_vec(&L.sbc, sbc));
   CK(upload_vec(&L.sbc_doff, L.sbc_off));
   // fields
@@ -2065,10 +2072,11 @@ static int smooth_core(Solve* s, int nl, int from_fine, int to_coarse, int niter
       // prim2cons_b; with the update folded into the CIRS sweep of a stage
       // that leaves q primitive, nothing reads the conservative state before
       // the sweep rewrites every interior cell from qold (and the next
-      // stage's BC fill rewrites the face halos), unless the HB or dual-time
-      // source takes it; on the last such stage the sweep writes the
-      // conservative interior, so only the face halos are converted
-      const bool fused_stage = fuse_update && iter <= niter && !c.harbal && !s->par.dualt;
+      // stage's halo fill every face halo, where it reads none: halo_fresh),
+      // unless the HB or dual-time source takes it; on the last such stage the
+      // sweep writes the conservative interior, so only the face halos are
+      // converted
+      const bool fused_stage = fuse_update && L.halo_fresh && iter <= niter && !c.harbal && !s->par.dualt;
       if (!(fused_stage && irk < c.nstage)) {
         TimeScope t(*s, COSAHIP_FAM_CONVERT, cs);
         CK(launch_prim2cons(*s, L, q, fused_stage));

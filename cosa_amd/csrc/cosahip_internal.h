@@ -244,7 +244,8 @@ struct Level {
   std::vector<Tile> hctile;   // cut work tiles (record, first item), records in order, and each record's first
   std::vector<int> ctile_first;
   Tile* ctile = nullptr;
-  bool halo_once = false;     // every face-halo cell set by one patch or cut point: k_halo may do all at once
+  bool halo_fresh = false;    // each halo fill sets every face-halo cell from interior cells (plan_halos)
+  bool halo_once = false;     // besides, every one by one patch or cut point: k_halo may do all at once
   bool thin = false;          // a block has < 2 cells in some direction
   // viscous / k-omega scratch
   double* vflux = nullptr;    // face fluxes (imax, jmax, kmax, npde, 0:2N), off_0 offsets; 3 slots

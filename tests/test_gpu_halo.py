@@ -76,3 +76,35 @@ def test_stages(open_face, nk):
         parity(g.download("q", 1), oc[1]["q"], what=f"q nk={nk} open={open_face}")
     finally:
         g.close()
+
+
+def _read_back_cases():
+    irs = {1: dict(irsop=1, cfl=1.0, cfl_irs=1.5), 2: dict(irsop=2, cfl=1.0, cfl_irs=1.5)}
+    two = dict(ni=9, nlevel=1, distort=0.2)
+    out = [cases.two_block_case(nj=9, nk=2, name=f"thin_symmetry_{m}", **two, **irs[m]) for m in irs]
+    out += [cases.two_block_case(nj=2, nk=5, name=f"thin_wall_{m}", **two, **irs[m]) for m in irs]
+    out += [cases.naca_case(33, 13, 2, nlevel=1, name=f"naca_2d_{m}", **irs[m]) for m in irs]
+    out.append(cases.two_block_case(nj=9, nk=2, wall=1500, name="thin_laminar", viscous=1, reyno=500.0, stemp=0.383,
+                                    **two, **irs[1]))
+    for m in irs:
+        c = cases.two_block_case(nj=9, nk=5, name=f"open_face_{m}", **two, **irs[m])
+        c.blocks[1].patches.pop()
+        out.append(Case(c.config, c.blocks, c.cuts, c.xyz, name=c.name))
+    return out
+
+
+@pytest.mark.parametrize("c", _read_back_cases(), ids=lambda c: c.name)
+def test_stages_that_read_halos(c):
+    """Smoothing with the RK update in the last sweep where a stage reads what
+    the stage before it left in a halo: symmetry planes and walls of a block
+    one cell thick (their second cell is the far halo) and a face that nothing
+    sets.  The conservative halos of prim2cons_b, as in the reference."""
+    q0 = c.perturbed(amp=0.01, seed=3)
+    o, oc, g = make_pair(c, q0)
+    try:
+        where, done = (ctypes.c_int32 * 8)(), (ctypes.c_int32 * 1)()
+        assert o.or_smooth(oc.ptr(), 1, 0, 0, 2, 1, done, where) == 0
+        g.smooth(1, False, False, 2, 1)
+        parity(g.download("q", 1), oc[1]["q"], what=f"q {c.name}")
+    finally:
+        g.close()
