@@ -1,0 +1,217 @@
+"""plan_halos (cosa_amd/csrc/halo_plan.h), which decides per level whether the
+halo fill may run as one launch and whether a smoothed stage may leave the
+halos as they are: against the cells that the BC patches (src/bc.f90) and cut
+copies (src/bc.f90:1894-2141) really read and write, over random faces, cut
+orientations and records that are no cut of two matching faces."""
+import ctypes
+import itertools
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cosa_amd", "csrc")
+
+HARNESS = """
+#include <cstdint>
+#include "halo_plan.h"
+struct Blk { int imax, jmax, kmax; };
+struct Patch { int block, type, t[10]; };
+struct Cut { int b1, b2, t[21]; };
+extern "C" int plan(int nb, const int* dims, int np, const int* pb, const int* pt, int nc, const int* ct) {
+  std::vector<Blk> b(nb);
+  std::vector<Patch> p(np);
+  std::vector<Cut> c(nc);
+  for (int m = 0; m < nb; m++) b[m] = Blk{dims[3 * m], dims[3 * m + 1], dims[3 * m + 2]};
+  for (int m = 0; m < np; m++) {
+    p[m].block = pb[m];
+    p[m].type = pt[10 * m];
+    std::copy(pt + 10 * m, pt + 10 * m + 10, p[m].t);
+  }
+  for (int m = 0; m < nc; m++) {
+    c[m].b1 = ct[21 * m] - 1;
+    c[m].b2 = ct[21 * m + 9] - 1;
+    std::copy(ct + 21 * m, ct + 21 * m + 21, c[m].t);
+  }
+  const cosahip::HaloPlan h = cosahip::plan_halos(b, p, c);
+  return h.fresh | h.once << 1;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    d = tmp_path_factory.mktemp("halo_plan")
+    (d / "h.cpp").write_text(HARNESS)
+    so = str(d / "h.so")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", CSRC, "-o", so, str(d / "h.cpp")])
+    return ctypes.CDLL(so)
+
+
+def cyc(d, m):
+    return (d - 1 + m - 1) % 3 + 1
+
+
+def _plan(lib, dims, patches, cuts):
+    a = [np.ascontiguousarray(x, np.int32).reshape(-1) for x in
+         (dims, [p[0] for p in patches], [p[1] for p in patches], cuts)]
+    p = [x.ctypes.data_as(ctypes.c_void_p) for x in a]
+    r = lib.plan(len(dims), p[0], len(patches), p[1], p[2], len(cuts), p[3])
+    return bool(r & 1), bool(r & 2)
+
+
+def cut_cells(dims, t):
+    """(block, halo cells set) and (block, cells read) of a record, the index
+    arithmetic of cut_q."""
+    d1, d2 = dims[t[0] - 1], dims[t[9] - 1]
+    i1, i2 = t[1], t[10]
+    iord = t[18:21]
+    ib, ibi = (0, -1) if t[2] == 1 else (d1[i1 - 1], 1)
+    inr, inri = (1, 1) if t[11] == 1 else (d2[i2 - 1] - 1, -1)
+    s1, e1 = [t[3 + 2 * m] for m in range(3)], [t[4 + 2 * m] for m in range(3)]
+    s2, e2 = [t[12 + 2 * m] for m in range(3)], [t[13 + 2 * m] for m in range(3)]
+    c1, c2, c3 = cyc(i1, 1) - 1, cyc(i1, 2) - 1, cyc(i1, 3) - 1
+    j1, j2, j3 = iord[c1] - 1, iord[c2] - 1, iord[c3] - 1
+
+    def sg(s, e, m):
+        return 1 if e[m] > s[m] else -1
+    to, frm = [], []
+    for a3, a2 in itertools.product(range(abs(e1[c3] - s1[c3]) + 1), range(abs(e1[c2] - s1[c2]) + 1)):
+        x, y = [0] * 3, [0] * 3
+        for ax, v in ((c1, ib), (c2, s1[c2] + sg(s1, e1, c2) * a2), (c3, s1[c3] + sg(s1, e1, c3) * a3)):
+            x[ax] += v
+        for ax, v in ((j1, inr), (j2, s2[j2] + sg(s2, e2, j2) * a2), (j3, s2[j3] + sg(s2, e2, j3) * a3)):
+            y[ax] += v
+        for m in (0, 1):
+            to.append(tuple(x[ax] + (m * ibi if ax == c1 else 0) for ax in range(3)))
+            frm.append(tuple(y[ax] + (m * inri if ax == j1 else 0) for ax in range(3)))
+    return (t[0] - 1, to), (t[9] - 1, frm)
+
+
+def patch_cells(dims, block, t):
+    d, i = dims[block], t[1] - 1
+    deep = t[0] not in (30, 4)   # walls and symmetry read two cells
+    out, frm = [], []
+    ax = [m for m in range(3) if m != i]
+    for a, b in itertools.product(*(range(t[3 + 2 * m], t[4 + 2 * m] + 1) for m in ax)):
+        for m in (0, 1):
+            x, y = [0] * 3, [0] * 3
+            x[ax[0]] = y[ax[0]] = a
+            x[ax[1]] = y[ax[1]] = b
+            x[i] = -m if t[2] == 1 else d[i] + m
+            y[i] = 1 + m if t[2] == 1 else d[i] - 1 - m
+            out.append(tuple(x))
+            if m == 0 or deep:
+                frm.append(tuple(y))
+    return (block, out), (block, frm)
+
+
+def expected(dims, patches, cuts):
+    moves = [patch_cells(dims, b, t) for b, t in patches] + [cut_cells(dims, t) for t in cuts]
+    inner = [set(itertools.product(*(range(1, n) for n in d))) for d in dims]
+    sets = [{} for _ in dims]
+    fresh = True
+    for (b, to), (b2, frm) in moves:
+        for x in to:
+            sets[b][x] = sets[b].get(x, 0) + 1
+        fresh &= all(y in inner[b2] for y in frm)
+    once = all(min(d) > 2 for d in dims)
+    for d, s in zip(dims, sets):
+        face = {x[:m] + (h,) + x[m:] for m in range(3)
+                for x in itertools.product(*(range(1, d[a]) for a in range(3) if a != m))
+                for h in (-1, 0, d[m], d[m] + 1)}
+        fresh &= face <= set(s)
+        once &= set(s) <= face and all(v == 1 for v in s.values())
+    return fresh, fresh and once
+
+
+def _in_p3(dims, t):
+    (b1, to), (b2, frm) = cut_cells(dims, t)
+    return all(-1 <= x <= n + 1 for b, cells in ((b1, to), (b2, frm)) for c in cells for x, n in zip(c, dims[b]))
+
+
+def _level(rng):
+    """Two blocks of the same cube, or one of another shape; every face a patch
+    or one side of a cut, some records then spoilt."""
+    n = int(rng.integers(2, 5))
+    dims = [[n + 1] * 3, [n + 1] * 3]
+    if rng.random() < 0.15:
+        dims[0][rng.integers(3)] = 2
+    faces = [(b, d, s) for b in (0, 1) for d in (1, 2, 3) for s in (0, 1)]
+    rng.shuffle(faces)
+    patches, cuts = [], []
+    rec = []
+    for b, d, s in [tuple(int(v) for v in f) for f in faces]:
+        lo, hi = [1, 1, 1], [v - 1 for v in dims[b]]
+        const = 1 if s == 0 else dims[b][d - 1]
+        lo[d - 1] = hi[d - 1] = const
+        rec.append((b, d, s, const, lo, hi))
+    while len(rec) >= 2 and rng.random() < 0.6:
+        f, g = rec.pop(), rec.pop()
+        for (b1, d1, _, k1, lo1, hi1), (b2, d2, _, k2, lo2, hi2) in ((f, g), (g, f)):
+            ta = [cyc(d2, 2), cyc(d2, 3)]
+            if rng.random() < 0.5:
+                ta.reverse()
+            iord = [0] * 3
+            iord[d1 - 1], iord[cyc(d1, 2) - 1], iord[cyc(d1, 3) - 1] = d2, *ta
+            r2 = [[lo2[m], hi2[m]] for m in range(3)]
+            for m in range(3):
+                if rng.random() < 0.5:
+                    r2[m].reverse()
+            t = [b1 + 1, d1, k1, *(v for m in range(3) for v in (lo1[m], hi1[m])),
+                 b2 + 1, d2, k2, *(v for r in r2 for v in r), *iord]
+            if all(hi1[cyc(d1, m) - 1] - lo1[cyc(d1, m) - 1] == abs(r2[iord[cyc(d1, m) - 1] - 1][1] -
+                   r2[iord[cyc(d1, m) - 1] - 1][0]) for m in (2, 3)):
+                cuts.append(t)
+    for b, d, _, const, lo, hi in rec:
+        patches.append((b, [int(rng.choice([30, 14, 80, 4])), d, const, *(v for m in range(3) for v in (lo[m], hi[m])), 0]))
+    spoilt = False
+    if rng.random() < 0.6 and cuts:
+        t = cuts[rng.integers(len(cuts))]
+        old = list(t)
+        for _ in range(int(rng.integers(1, 4))):
+            m = int(rng.integers(12, 21))
+            t[m] = int(rng.integers(1, 4)) if m >= 18 else int(rng.integers(1, n + 2))
+        if _in_p3(dims, t):
+            spoilt = t != old
+        else:
+            t[:] = old
+    elif rng.random() < 0.2 and patches:
+        patches.pop()
+    return dims, patches, cuts, spoilt
+
+
+def test_against_the_cells_read_and_set(lib):
+    rng = np.random.default_rng(0)
+    seen = set()
+    for m in range(6000):
+        dims, patches, cuts, spoilt = _level(rng)
+        got, want = _plan(lib, dims, patches, cuts), expected(dims, patches, cuts)
+        # a record that is no cut may be refused though it would do no harm
+        assert got == want or (spoilt and got[0] <= want[0] and got[1] <= want[1]), (m, dims, patches, cuts, got, want)
+        seen.add((got, spoilt))
+    assert {((True, True), False), ((False, False), False), ((False, False), True), ((True, False), False)} <= seen
+
+
+def test_order_that_disagrees_with_the_face(lib):
+    """A record whose index order does not map the normal of face 1 to the
+    normal of face 2: the cells it reads lie along another axis of block 2, in
+    its halo where that axis is shorter."""
+    dims = [[4, 4, 4], [4, 3, 4]]
+    full = [[1, 3, 1, 3, 1, 3], [1, 3, 1, 2, 1, 3]]
+    patches = []
+    for b in (0, 1):
+        for d in (1, 2, 3):
+            for k in (1, dims[b][d - 1]):
+                if (b, d, k) == (0, 1, 4):
+                    continue
+                r = list(full[b])
+                r[2 * d - 2] = r[2 * d - 1] = k
+                patches.append((b, [30, d, k, *r, 0]))
+    # face i = imax of block 1 from the i = imax side of block 2, order (2, 1, 3):
+    # cell imax - 1 = 3 of block 2 is taken along j, where the halo starts at 3
+    cut = [1, 1, 4, 4, 4, 1, 3, 1, 3, 2, 1, 4, 1, 3, 1, 3, 1, 3, 2, 1, 3]
+    assert _in_p3(dims, cut)
+    assert not expected(dims, patches, [cut])[0]
+    assert _plan(lib, dims, patches, [cut]) == (False, False)
