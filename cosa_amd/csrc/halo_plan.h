@@ -9,6 +9,51 @@
 
 namespace cosahip {
 
+// Host replica of k_cut's index arithmetic: every halo target and interior
+// source of the cut must lie inside its block's P3 extents.
+template <class Block>
+bool cut_in_bounds(const Block& b1, const Block& b2, const int* t, int n2, int count) {
+  const int idir1 = t[1], inout1 = t[2], idir2 = t[10], inout2 = t[11];
+  int istr1[4], iend1[4], istr2[4], iend2[4], iord[4];
+  istr1[1] = t[3]; iend1[1] = t[4]; istr1[2] = t[5]; iend1[2] = t[6]; istr1[3] = t[7]; iend1[3] = t[8];
+  istr2[1] = t[12]; iend2[1] = t[13]; istr2[2] = t[14]; iend2[2] = t[15]; istr2[3] = t[16]; iend2[3] = t[17];
+  iord[1] = t[18]; iord[2] = t[19]; iord[3] = t[20];
+  for (int m = 1; m <= 3; m++)
+    if (iord[m] < 1 || iord[m] > 3) return false;
+  const int ijk1[4] = {0, b1.imax, b1.jmax, b1.kmax}, ijk2[4] = {0, b2.imax, b2.jmax, b2.kmax};
+  const int ibcpt = inout1 == 1 ? 0 : ijk1[idir1], ibcinc = inout1 == 1 ? -1 : 1;
+  const int inr = inout2 == 1 ? 1 : ijk2[idir2] - 1, inrinc = inout2 == 1 ? 1 : -1;
+  auto cyc = [](int d, int m) { return (d - 1 + m - 1) % 3 + 1; };
+  const int ic1 = cyc(idir1, 1), ic2 = cyc(idir1, 2), ic3 = cyc(idir1, 3);
+  const int jc1 = iord[ic1], jc2 = iord[ic2], jc3 = iord[ic3];
+  const int sg1c2 = iend1[ic2] > istr1[ic2] ? 1 : -1, sg1c3 = iend1[ic3] > istr1[ic3] ? 1 : -1;
+  const int sg2c2 = iend2[jc2] > istr2[jc2] ? 1 : -1, sg2c3 = iend2[jc3] > istr2[jc3] ? 1 : -1;
+  auto inside = [](const Block& b, int i, int j, int k) {
+    return i >= -1 && i <= b.imax + 1 && j >= -1 && j <= b.jmax + 1 && k >= -1 && k <= b.kmax + 1;
+  };
+  for (int item = 0; item < count; item++) {
+    const int i2_ = item % n2, i3_ = item / n2;
+    const int a2 = istr1[ic2] + sg1c2 * i2_, a3 = istr1[ic3] + sg1c3 * i3_;
+    int x1[4] = {0, 0, 0, 0};
+    x1[ic1] = ibcpt;
+    x1[ic2] = a2;
+    x1[ic3] = a3;
+    int x2[4] = {0, x1[1], x1[2], x1[3]};
+    x2[ic1] += ibcinc;
+    const int c2 = istr2[jc2] + sg2c2 * i2_, c3 = istr2[jc3] + sg2c3 * i3_;
+    int y1[4] = {0, 0, 0, 0};
+    y1[jc1] += inr;   // sums, as in bc_ijk, where the order repeats an axis
+    y1[jc2] += c2;
+    y1[jc3] += c3;
+    int y2[4] = {0, y1[1], y1[2], y1[3]};
+    y2[jc1] += inrinc;
+    if (!inside(b1, x1[1], x1[2], x1[3]) || !inside(b1, x2[1], x2[2], x2[3]) || !inside(b2, y1[1], y1[2], y1[3]) ||
+        !inside(b2, y2[1], y2[2], y2[3]))
+      return false;
+  }
+  return true;
+}
+
 // What the halo fill of a level may be relied on for.
 // fresh: every face-halo cell of every block is set by each fill, from
 // interior cells alone.  A wall, symmetry or cut record reads two cells deep,

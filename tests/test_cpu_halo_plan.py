@@ -1,6 +1,6 @@
-"""plan_halos (cosa_amd/csrc/halo_plan.h), which decides per level whether the
-halo fill may run as one launch and whether a smoothed stage may leave the
-halos as they are: against the cells that the BC patches (src/bc.f90) and cut
+"""The host checks of halo_plan.h -- plan_halos, which decides per level
+whether the halo fill may run as one launch and whether a smoothed stage may
+leave the halos as they are, and cut_in_bounds: against the cells that the BC patches (src/bc.f90) and cut
 copies (src/bc.f90:1894-2141) really read and write, over random faces, cut
 orientations and records that are no cut of two matching faces."""
 import ctypes
@@ -36,6 +36,11 @@ extern "C" int plan(int nb, const int* dims, int np, const int* pb, const int* p
   }
   const cosahip::HaloPlan h = cosahip::plan_halos(b, p, c);
   return h.fresh | h.once << 1;
+}
+extern "C" int in_bounds(const int* d1, const int* d2, const int* t) {
+  const int i2 = t[1] % 3 + 1, i3 = (t[1] + 1) % 3 + 1;
+  const int l2 = std::abs(t[2 * i2 + 2] - t[2 * i2 + 1]) + 1, l3 = std::abs(t[2 * i3 + 2] - t[2 * i3 + 1]) + 1;
+  return cosahip::cut_in_bounds(Blk{d1[0], d1[1], d1[2]}, Blk{d2[0], d2[1], d2[2]}, t, l2, l2 * l3);
 }
 """
 
@@ -215,3 +220,20 @@ def test_order_that_disagrees_with_the_face(lib):
     assert _in_p3(dims, cut)
     assert not expected(dims, patches, [cut])[0]
     assert _plan(lib, dims, patches, [cut]) == (False, False)
+
+
+def test_cut_in_bounds(lib):
+    """Records that reach outside either block's array are refused, also where
+    the order names an axis twice and its indices add up."""
+    rng = np.random.default_rng(1)
+    seen = {False: 0, True: 0}
+    for _ in range(6000):
+        dims = rng.integers(2, 6, (2, 3)).tolist()
+        t = [1, int(rng.integers(1, 4)), int(rng.integers(1, 3)), *rng.integers(0, 6, 6).tolist(),
+             2, int(rng.integers(1, 4)), int(rng.integers(1, 3)), *rng.integers(-1, 6, 6).tolist(),
+             *rng.integers(1, 4, 3).tolist()]
+        a = [np.array(x, np.int32) for x in (*dims, t)]
+        got = bool(lib.in_bounds(*(x.ctypes.data_as(ctypes.c_void_p) for x in a)))
+        assert got == _in_p3(dims, t), (dims, t)
+        seen[got] += 1
+    assert min(seen.values()) > 100
