@@ -15,7 +15,11 @@ from parity_util import TURB
 
 pytestmark = pytest.mark.gpu
 
-SMALL = [(34, 18, 6), (9, 2, 3), (17, 12, 40), (71, 37, 15)]
+# A channel one cell high is not among them: its walls extrapolate from the far
+# halo, which holds conservative values, and the reference's scheme fails the
+# positivity test there (9 x 2 x 3 nodes: oracle and GPU at cell (1, -1, 1) of
+# the second stage, any irsop); test_one_cell_j_lines has farfields there.
+SMALL = [(34, 18, 6), (9, 3, 2), (17, 12, 40), (71, 37, 15)]
 LONG = [(4, 330, 3), (3, 5, 420), (1100, 3, 4)]
 TOO_LONG = [(3, 620, 4), (1600, 3, 3)]
 IRS = {1: dict(irsop=1, cfl=2.0, cfl_irs=4.0), 2: dict(irsop=2, cfl=2.0, cfl_irs=4.0)}
@@ -51,6 +55,12 @@ def _compare(c, monkeypatch):
 @pytest.mark.parametrize("dims", [SMALL, LONG, TOO_LONG], ids=["small", "long", "too_long"])
 def test_euler_same_bits(dims, irsop, monkeypatch):
     _compare(cases.channel_case(dims, nlevel=1, name=f"channels_{irsop}", **IRS[irsop]), monkeypatch)
+
+
+@pytest.mark.parametrize("irsop", [1, 2])
+def test_one_cell_j_lines(irsop, monkeypatch):
+    _compare(cases.two_block_case(ni=9, nj=2, nk=4, nlevel=1, distort=0.1, wall=30, name=f"flat_{irsop}",
+                                  **IRS[irsop]), monkeypatch)
 
 
 @pytest.mark.parametrize("irsop", [1, 2])
