@@ -406,7 +406,8 @@ static void plan_cirs_il(Solve* s, Level& L) {
     lmax = std::max(lmax, B.imax - 1);
     lines += (ll)s->par.nsnap * (B.jmax - 1) * (B.kmax - 1);
   }
-  const ll S = lmax | 1, tab = s->par.irsop == 1 ? 16 * S + 8 : 0, row = 8 * S * cirs_strip_per(s->par);
+  const bool cc = s->par.irsop == 1;
+  const ll S = lmax | 1, tab = cc ? 16 * S + 8 : 0, row = 8 * S * cirs_strip_per(s->par.npde, cc);
   if (tab + row > 79000) return;
   ll lpw = std::max<ll>(1, (s->il_lds - tab) / row);
   lpw = std::min(lpw, std::min<ll>(256 / s->par.npde, (lines + 511) / 512));
@@ -418,19 +419,18 @@ static void plan_cirs_il(Solve* s, Level& L) {
 // k_cirs_strip: LDS bytes of a work-group per direction, the largest over the
 // blocks; 0 (the line kernels instead) when some block's line does not fit.
 static void plan_cirs_strip(Solve* s, Level& L) {
-  const int per = cirs_strip_per(s->par), nv = s->par.npde;
+  const int nv = s->par.npde;
+  const bool cc = s->par.irsop == 1;
   for (int d = 0; d < 2; d++) {
     L.strip_lds[d] = 0;
     if (s->par.irsop < 1 || s->cirs_jk_mode != 2) continue;
     for (const Blk& b : L.hblk) {
-      const int n = (d == 0 ? b.jmax : b.kmax) - 1, w = cirs_strip_w(n, b.imax - 1, per);
+      const int n = (d == 0 ? b.jmax : b.kmax) - 1, w = cirs_strip_w(n, b.imax - 1, nv, cc);
       if (!w || n >= JK_RT) {
         L.strip_lds[d] = 0;
         break;
       }
-      const size_t bytes = sizeof(double) * ((size_t)nv * cirs_strip_vs(n, w) +
-                                             (s->par.irsop == 1 ? 2 * (size_t)n + 1 : (size_t)(per - nv) * n * w));
-      L.strip_lds[d] = std::max(L.strip_lds[d], bytes);
+      L.strip_lds[d] = std::max(L.strip_lds[d], (size_t)cirs_strip_lds(n, w, nv, cc));
     }
   }
 }
@@ -517,7 +517,7 @@ static int build_tables(Solve* s, Level& L, const Level* Lc) {
     if (L.il_lpw) add_tiles(L.htile[TK_LINES_IL], b, ns * jm * km, L.il_lpw);
     for (int d = 0; d < 2; d++)
       if (L.strip_lds[d]) {
-        const int w = cirs_strip_w((int)(d == 0 ? jm : km), (int)im, cirs_strip_per(s->par));
+        const int w = cirs_strip_w((int)(d == 0 ? jm : km), (int)im, s->par.npde, s->par.irsop == 1);
         add_tiles(L.htile[d == 0 ? TK_STRIP_J : TK_STRIP_K], b, ns * ((im + w - 1) / w) * (d == 0 ? km : jm), 1);
       }
     if (s->par.viscous) {

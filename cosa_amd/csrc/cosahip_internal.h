@@ -109,23 +109,36 @@ enum TileKind {
   TK_NKIND
 };
 
-// k_cirs_strip: lines (cells along i) of one work-group for lines of L cells
-// in a block im cells wide, per = doubles of LDS per cell of a line.  A power
-// of two; whole lines stay within 40 KB, so that three or four work-groups
-// share a CU, as long as that leaves 8 (a 64-byte run in memory); longer
-// lines keep 8 up to the LDS of half a CU and then 4.  0: the line does not fit.
-__host__ __device__ inline int cirs_strip_w(int L, int im, int per) {
-  int w = 32;   // 32 x 7 variables fit the threads of a work-group
-  while (w > 8 && ((ll)w * L * per * 8 > 40960 || w >= 2 * im)) w >>= 1;
-  if ((ll)w * L * per * 8 > 79000) w = 4;
-  return (ll)w * L * per * 8 > 79000 ? 0 : w;
-}
-// doubles of LDS per cell: the variables and, with variable coefficients, the
-// coefficient and multiplier of the mean flow and of k-omega
-inline int cirs_strip_per(const Par& p) { return p.npde + (p.irsop == 1 ? 0 : p.npde > 5 ? 4 : 2); }
-// LDS stride of one variable's strip in doubles: the variables' lanes of a
-// half-wave fall into different banks
+// LDS stride of one variable's strip of k_cirs_strip in doubles: the variables'
+// lanes of a half-wave fall into different banks
 __host__ __device__ inline int cirs_strip_vs(int L, int w) { return w < 32 ? ((L * w + 31) & ~31) + w : L * w; }
+// doubles of LDS per cell: the nv variables and, with variable coefficients
+// (cc false), the coefficient and multiplier of the mean flow and of k-omega
+__host__ __device__ inline int cirs_strip_per(int nv, bool cc) { return nv + (cc ? 0 : nv > 5 ? 4 : 2); }
+// LDS bytes of a work-group: the padded strips, then the block's table or the
+// coefficients and multipliers of every line
+__host__ __device__ inline ll cirs_strip_lds(int L, int w, int nv, bool cc) {
+  return 8 * ((ll)nv * cirs_strip_vs(L, w) + (cc ? 2 * (ll)L + 1 : (ll)(cirs_strip_per(nv, cc) - nv) * L * w));
+}
+// k_cirs_strip: lines (cells along i) of one work-group for lines of L cells
+// in a block im cells wide.  A power of two; whole lines stay within 40 KB, so
+// that three or four work-groups share a CU, as long as that leaves 8 (a
+// 64-byte run in memory); longer lines keep 8 while two work-groups share a CU
+// (80 KB each) and then 4, to 79000 bytes of line: alone on a CU from 458
+// cells, and still twice as fast as the line kernels.  0: the line does not fit.
+// All three sweeps of 2.4 M cells, us, j-lines of L cells (k-lines are alike),
+// the line kernels (irsop 1: k_cirs_jkc) -> this rule:
+//   mean flow, irsop 1   L 128: 545 -> 247, 256: 497 -> 247, 352: 548 -> 273, 448: 616 -> 259, 492: 653 -> 341
+//   mean flow, irsop 2   128: 813 -> 358, 256: 722 -> 365, 352: 790 -> 372
+//   k-omega, irsop 1     128: 632 -> 325, 240: 576 -> 322, 352: 642 -> 400
+//   k-omega, irsop 2     176: 1314 -> 626, 208: 1288 -> 585
+__host__ __device__ inline int cirs_strip_w(int L, int im, int nv, bool cc) {
+  const ll cell = 8 * cirs_strip_per(nv, cc);
+  int w = 32;   // 32 x 7 variables fit the threads of a work-group
+  while (w > 8 && (w * L * cell > 40960 || w >= 2 * im)) w >>= 1;
+  if (cirs_strip_lds(L, w, nv, cc) > 81920) w = 4;
+  return w == 4 && w * L * cell > 79000 ? 0 : w;
+}
 
 // inviscid residual kernels (the same bits; chosen per level by
 // cosahip_autotune or COSAHIP_RESIDUAL at create time)

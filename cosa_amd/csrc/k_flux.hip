@@ -1157,7 +1157,7 @@ __global__ void __launch_bounds__(256) k_cirs_strip(Par p, const Blk* __restrict
   const Blk b = blks[t.block];
   const int im = b.imax - 1, jm = b.jmax - 1, km = b.kmax - 1;
   const int L = DIR == 2 ? jm : km, T2 = DIR == 2 ? km : jm;
-  const int W = cirs_strip_w(L, im, NV + (CC ? 0 : 2 * NG)), VS = cirs_strip_vs(L, W);
+  const int W = cirs_strip_w(L, im, NV, CC), VS = cirs_strip_vs(L, W);
   const int nst = (im + W - 1) / W;
   int item = t.base;
   const int n = item / (nst * T2);
