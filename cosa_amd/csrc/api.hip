@@ -273,7 +273,9 @@ int cosahip_create(const cosahip_config* cfg, int device, cosahip_solve** out) {
   const char* gk = getenv("COSAHIP_GRAPH");
   s->use_graph = !(gk && strcmp(gk, "0") == 0);
   const char* ck = getenv("COSAHIP_CIRS_I");
-  s->cirs_i_mode = !ck ? 0 : strcmp(ck, "lds") == 0 || strcmp(ck, "iv") == 0 ? 2 : strcmp(ck, "line") == 0 ? 3 : 0;
+  s->cirs_i_mode = !ck ? 0 : strcmp(ck, "iv") == 0 ? 2 : strcmp(ck, "line") == 0 ? 3 : 0;
+  if (ck && !s->cirs_i_mode)
+    fprintf(stderr, "cosahip_create: COSAHIP_CIRS_I=%s is not one of iv, line: the i-sweep is chosen per level\n", ck);
   const char* lk = getenv("COSAHIP_CIRS_IL_LDS");
   if (lk) s->il_lds = std::min(65536, std::max(4096, atoi(lk)));
   const char* vk = getenv("COSAHIP_VISCOUS");

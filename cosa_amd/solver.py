@@ -301,7 +301,7 @@ class Solve:
         and keep the fastest (cosahip_autotune); results are unchanged."""
         ch = (ctypes.c_int32 * 8)()
         self._check(self.lib.cosahip_autotune(self.h, reps, ch), "autotune")
-        names = {0: None, 1: "lds", 2: "per_variable", 3: "line_resident"}
+        names = {0: None, 2: "per_variable", 3: "line_resident"}
         rnames = {-1: None, 0: "generic_fused", 1: "tile31x7", 2: "tile31x7_register_window", 3: "tile31x15",
                   4: "tile31x7_128vgpr", 5: "tile31x7_shared_slopes", 6: "tile31x15_shared_slopes",
                   7: "tile31x7_shared_slopes_128vgpr", 8: "tile32x7_128vgpr", 9: "tile32x7_shared_slopes"}

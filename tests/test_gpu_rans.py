@@ -236,14 +236,14 @@ def test_viscous_tile_pass_matches(c, prec, monkeypatch):
 
 def test_cirs_i_variants_agree(monkeypatch):
     """CIRS i-sweep: one thread per (line, variable) with k and omega in the
-    same launch (COSAHIP_CIRS_I=iv, the default on small levels) and one
-    thread per line with LDS-staged chunks (COSAHIP_CIRS_I=lds) give
-    bit-identical results."""
+    same launch (COSAHIP_CIRS_I=iv) and whole lines resident in LDS
+    (COSAHIP_CIRS_I=line) give bit-identical results with variable
+    coefficients (irsop 2 and 3)."""
     from cosa_amd.solver import Solve
     for c in (CASES[0], CASES[2]):
         q0 = c.perturbed(amp=0.02, seed=17)
         res = []
-        for mode in ("iv", "lds"):
+        for mode in ("iv", "line"):
             monkeypatch.setenv("COSAHIP_CIRS_I", mode)
             g = Solve(c, device=0, q=q0)
             try:
@@ -252,6 +252,27 @@ def test_cirs_i_variants_agree(monkeypatch):
             finally:
                 g.close()
         assert np.array_equal(res[0], res[1]), c.name
+
+
+def test_cirs_i_unknown_variant(monkeypatch, capfd):
+    """A sweep that does not exist is named on stderr and the level's own
+    choice is taken."""
+    from cosa_amd.solver import Solve
+    c = CASES[0]
+    q0 = c.perturbed(amp=0.02, seed=17)
+    res = []
+    for mode in (None, "lds"):
+        if mode:
+            monkeypatch.setenv("COSAHIP_CIRS_I", mode)
+        capfd.readouterr()
+        g = Solve(c, device=0, q=q0)
+        try:
+            assert ("COSAHIP_CIRS_I=lds" in capfd.readouterr().err) == (mode == "lds")
+            g.smooth(1, False, False, 2, 1)
+            res.append(g.download("q"))
+        finally:
+            g.close()
+    assert np.array_equal(res[0], res[1])
 
 
 def _irsop1_cases():
