@@ -169,20 +169,18 @@ def test_rans_multigrid_cycles(name):
 
 
 def test_viscous_kernel_variants_agree(monkeypatch):
-    """The three arrangements of the viscous face work give bit-identical
-    residuals (same operands, same accumulation order): face fluxes stored
-    then differenced (default), flux and difference in one marching kernel
-    (COSAHIP_VISCOUS=march), fused into the inviscid line march
-    (COSAHIP_VISCOUS=fused)."""
+    """The arrangements of the viscous face work give bit-identical residuals
+    (same operands, same accumulation order): face fluxes stored then
+    differenced per direction (COSAHIP_VISCOUS=faces), flux and difference in
+    one marching kernel (march), fused into the inviscid line march (fused),
+    and the fluxes of all three directions stored, then differenced in one tile
+    pass with the inviscid fluxes (tile, the default)."""
     from cosa_amd.solver import Solve
     c = CASES[0]
     q0 = c.perturbed(amp=0.02, seed=13)
     out = []
-    for mode in ("default", "fused", "march", "tile"):
-        if mode == "default":
-            monkeypatch.delenv("COSAHIP_VISCOUS", raising=False)
-        else:
-            monkeypatch.setenv("COSAHIP_VISCOUS", mode)
+    for mode in ("faces", "fused", "march", "tile"):
+        monkeypatch.setenv("COSAHIP_VISCOUS", mode)
         g = Solve(c, device=0, q=q0)
         try:
             for f in ("cons2prim", "bc", "cutman_q"):
@@ -205,21 +203,18 @@ def _tile_pass_cases():
 @pytest.mark.parametrize("prec", [0, 1], ids=["fp64", "fp32res"])
 @pytest.mark.parametrize("c", _tile_pass_cases(), ids=lambda c: c.name)
 def test_viscous_tile_pass_matches(c, prec, monkeypatch):
-    """The tile arrangement (COSAHIP_VISCOUS=tile: viscous face fluxes of
-    the three directions stored, then one 31 x 7 tile pass forming the
-    inviscid fluxes of every direction and summing them with the viscous
-    differences in the reference's order) leaves the same bits as the
-    default per-direction kernels after two smoothing iterations, in FP64
-    and in the FP32-residual mode (laminar, Wilcox, Menter BSL / SST,
-    harmonic balance, the NACA O-grid with tiles that overhang the block)."""
+    """The tile arrangement (the default: viscous face fluxes of the three
+    directions stored, then one pass over 32 x 7 tiles forming the inviscid
+    fluxes of every direction and summing them with the viscous differences in
+    the reference's order) leaves the same bits as the per-direction kernels
+    (COSAHIP_VISCOUS=faces) after two smoothing iterations, in FP64 and in the
+    FP32-residual mode (laminar, Wilcox, Menter BSL / SST, harmonic balance,
+    the NACA O-grid with tiles that overhang the block)."""
     from cosa_amd.solver import Solve
     q0 = c.perturbed(amp=0.02, seed=23)
     out = []
-    for mode in (None, "tile"):
-        if mode is None:
-            monkeypatch.delenv("COSAHIP_VISCOUS", raising=False)
-        else:
-            monkeypatch.setenv("COSAHIP_VISCOUS", mode)
+    for mode in ("faces", "tile"):
+        monkeypatch.setenv("COSAHIP_VISCOUS", mode)
         g = Solve(c, device=0, q=q0)
         try:
             if prec:
