@@ -507,7 +507,7 @@ static int build_tables(Solve* s, Level& L, const Level* Lc) {
     const Blk& B = L.hblk[b];
     const ll im = B.imax - 1, jm = B.jmax - 1, km = B.kmax - 1;
     add_tiles(L.htile[TK_CELLS], b, ns * im * jm * km, TS);
-    if (s->cfg.harbal && ns >= 3 && ns <= 9) add_tiles(L.htile[TK_CELLV], b, s->par.npde * im * jm * km, TS);
+    if (s->cfg.harbal && src_hbv_has(ns)) add_tiles(L.htile[TK_CELLV], b, s->par.npde * im * jm * km, TS);
     const ll nseg = (im + ROWSEG - 1) / ROWSEG;
     add_tiles(L.htile[TK_ROWS_I], b, ns * jm * km * nseg, 4);
     add_tiles(L.htile[TK_LINES_J], b, ns * im * km, TS);

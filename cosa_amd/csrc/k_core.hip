@@ -532,8 +532,9 @@ __global__ void __launch_bounds__(256) k_src_hb(Par p, const Blk* __restrict__ b
 // The same with a thread for a cell and variable of all NS snapshots: it loads
 // the NS states once, where a thread of k_src_hb loads them all for one
 // snapshot's source, NS times over, one variable after another.  For up to 4
-// harmonics (TK_CELLV); above, the unrolled NS x NS sums no longer fit the
-// registers.  147456 cells x 9
+// harmonics (src_hbv_has): the unrolled sums hold the matrix in scalar
+// registers, all of it at 9 snapshots (102 VGPRs); at 11, 13 and 17 they spill
+// 240, 304 and 576 of them.  147456 cells x 9
 // snapshots: 84 -> 39 us against k_src_hb (5.4 TB/s).
 template <int NS>
 __global__ void __launch_bounds__(256) k_src_hbv(Par p, const Blk* __restrict__ blks, const Tile* __restrict__ tiles,
@@ -1621,20 +1622,20 @@ hipError_t launch_update(Solve& s, Level& L, double ar, const UpdateTail& up) {
   return hipGetLastError();
 }
 hipError_t launch_src_hb(Solve& s, Level& L) {
-  if (L.ntile[TK_CELLV]) {
-    const dim3 g = grid1(L.ntile[TK_CELLV]);
-    auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, g, dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLV], L.f[COSAHIP_Q],
-                         L.f[COSAHIP_VOL], L.f[COSAHIP_RES], L.dq, s.ddhb);
-    };
-    if (s.par.nsnap == 3) go(k_src_hbv<3>);
-    else if (s.par.nsnap == 5) go(k_src_hbv<5>);
-    else if (s.par.nsnap == 7) go(k_src_hbv<7>);
-    else go(k_src_hbv<9>);
-  } else if (L.ntile[TK_CELLS]) {
-    // one work item per interior (cell, snapshot)
-    hipLaunchKernelGGL(k_src_hb, grid1(L.ntile[TK_CELLS]), dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLS],
-                       L.f[COSAHIP_Q], L.f[COSAHIP_VOL], L.f[COSAHIP_RES], L.dq, s.ddhb);
+  auto go = [&](auto kernel) {
+    if (L.ntile[TK_CELLV])
+      hipLaunchKernelGGL(kernel, grid1(L.ntile[TK_CELLV]), dim3(TS), 0, s.stream, s.par, L.dblk, L.tile[TK_CELLV],
+                         L.f[COSAHIP_Q], L.f[COSAHIP_VOL], L.f[COSAHIP_RES], L.dq, s.ddhb);
+  };
+  switch (s.par.nsnap) {   // src_hbv_has
+    case 3: go(k_src_hbv<3>); break;
+    case 5: go(k_src_hbv<5>); break;
+    case 7: go(k_src_hbv<7>); break;
+    case 9: go(k_src_hbv<9>); break;
+    default:   // one work item per interior (cell, snapshot)
+      if (L.ntile[TK_CELLS])
+        hipLaunchKernelGGL(k_src_hb, grid1(L.ntile[TK_CELLS]), dim3(TS), 0, s.stream, s.par, L.dblk,
+                           L.tile[TK_CELLS], L.f[COSAHIP_Q], L.f[COSAHIP_VOL], L.f[COSAHIP_RES], L.dq, s.ddhb);
   }
   return hipGetLastError();
 }

@@ -35,6 +35,8 @@ hipError_t launch_rms_hb_term(Solve& s, Level& L, double* work1);
 hipError_t launch_src_uns(Solve& s, Level& L, int sub_rhs);
 hipError_t launch_rhs_uns(Solve& s, Level& L);
 hipError_t launch_rms_dual_term(Solve& s, Level& L, double* work1);
+// snapshot counts that k_src_hbv is built for (the others: k_src_hb); they take the TK_CELLV tiles
+inline bool src_hbv_has(int nsnap) { return nsnap == 3 || nsnap == 5 || nsnap == 7 || nsnap == 9; }
 hipError_t launch_src_hb(Solve& s, Level& L);
 hipError_t launch_rms(Solve& s, Level& L, const double* res, const double* rhs, int use_rhs);
 hipError_t launch_prtest(Solve& s, Level& L, const double* q, int stage_seq);
