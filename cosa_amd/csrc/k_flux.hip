@@ -1136,7 +1136,8 @@ __device__ __forceinline__ void strip_back(double* __restrict__ x, const double*
 // and one write of res (UPD: q written instead, qold and the time step read)
 // where the chunked sweep read res twice; a thread's recurrence waits on LDS
 // instead of HBM.  Level 1 of 48 uneven blocks (11.8 M cells): j 455 -> 329
-// us, k with the update 673 -> 505; 128 x 33 x 5 O-grids and SST j-lines with
+// us, k with the update 673 -> 505 (256 and 428 since neighbouring strips share
+// an XCD, xcd_order); 128 x 33 x 5 O-grids and SST j-lines with
 // variable coefficients 135 -> 24.  Narrower strips or 20 KB were no faster.
 // CC: the constant coefficient of irsop 1, multipliers r(a) and reciprocal
 // divisors from the block's table; else each thread forms r(a) from the

@@ -576,7 +576,11 @@ ll residual_tile_items(int TI, int TJ, int kseg, int imax, int jmax, int kmax, i
 // segments -> this rule): one 17^3-node block 109 -> 14, the 193 x 49 x 9
 // O-grid 63 -> 21, 97 x 49 x 49 nodes 234 -> 36, 48 uneven blocks 1382 -> 1270
 // on level 1 and 284 -> 146 on level 2; over 17 levels of ten grids the
-// pick is within 5% of the best of 1, 2, 3, 4, 6, 8, 12, 16, 32.
+// pick is within 5% of the best of 1, 2, 3, 4, 6, 8, 12, 16, 32.  The
+// constants are those of the FP64 second-order kernel, but hold for the others
+// too: second and first order, limiter 1, FP32, contracted, laminar, k-omega
+// (FP64 and FP32) and SST residuals on ten levels of 4096 to 2.1 M cells are
+// within 7% of their best of 1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 68 of the 90 within 1%.
 int residual_kseg(const std::vector<Blk>& blks, int nsnap) {
   int best = RT_KSEG;
   double tbest = 0;

@@ -20,8 +20,9 @@ namespace cosahip {
 // The bits are those of the division and the root for operands without
 // extreme exponents (states and their differences: no subnormals, no
 // overflow; below 1e-290 a quotient keeps its absolute, not its relative
-// rounding).  A zero or negative divisor, where the flow state has failed
-// already, gives NaN where the division gives an infinity.
+// rounding).  Where the flow state has failed already they give NaN: for a zero
+// or negative divisor, for which the division gives an infinity, and for an
+// infinite operand, for which division, root and power give an infinity or zero.
 // FP32 and the contracted build use the operators.
 // Residual of 48 uneven blocks (with the end tests of muscl_face below):
 // VALU instructions 439 M -> 334 M, level 1 1230 -> 1128 us, level 2 160 -> 133;
