@@ -21,8 +21,8 @@ pytestmark = pytest.mark.gpu
 # the second stage, any irsop); test_one_cell_j_lines has farfields there.
 SMALL = [(34, 18, 6), (9, 3, 2), (17, 12, 40), (71, 37, 15)]
 LONG = [(4, 330, 3), (3, 5, 420), (1100, 3, 4)]
-# j / k lines at the half-CU bound of 8 lines a work-group, its table and padding counted
-EDGE = [(9, 242, 3), (5, 3, 243), (11, 247, 4), (7, 178, 3), (6, 3, 177)]
+# j / k lines at the half-CU bound of 8 lines a work-group, its table and padding counted, and the longest for 4
+EDGE = [(9, 242, 3), (5, 3, 243), (11, 247, 4), (7, 178, 3), (6, 3, 177), (4, 3, 493)]
 TOO_LONG = [(3, 620, 4), (1600, 3, 3)]
 IRS = {1: dict(irsop=1, cfl=2.0, cfl_irs=4.0), 2: dict(irsop=2, cfl=2.0, cfl_irs=4.0)}
 
@@ -72,7 +72,7 @@ def test_komega_same_bits(irsop, monkeypatch):
                                   **kw_turbulence(0.5, 1e5, tu=1e-3, mutfar=0.1, **TURB)), monkeypatch)
 
 
-@pytest.mark.parametrize("nj", [173, 174, 178])
+@pytest.mark.parametrize("nj", [173, 174, 178, 353])
 def test_komega_edge_same_bits(nj, monkeypatch):
     kw = dict(irsop=1, cfl=1.5, cfl_irs=2.5, ratt=1.4, cflt=1.2)
     _compare(cases.two_block_case(ni=6, nj=nj, nk=4, nlevel=1, distort=0.1, name=f"komega_{nj}", wall=1500, **kw,
