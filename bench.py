@@ -81,8 +81,8 @@ BYTES_PER_CELL_RANS = {  # Wilcox k-omega, npde = 7
 # profiles/residual_uneven96_fp64_hbm_traffic.md
 # and profiles/residual_wing4_rans_fp64_hbm_traffic.md.  Re-measure when the
 # kernels change.
-MEASURED_TRAFFIC_PER_CELL = {("uneven96", "fp64", "residual"): 256.7, ("uneven96", "fp64", "cirs"): 351.6,
-                             ("wing4", "fp64", "residual"): 2109.7}
+MEASURED_TRAFFIC_PER_CELL = {("uneven96", "fp64", "residual"): 256.6, ("uneven96", "fp64", "cirs"): 351.6,
+                             ("wing4", "fp64", "residual"): 2109.9}
 
 
 def log(msg):
